@@ -143,6 +143,17 @@ LevelDesc make_level_desc(const mfs_box &b, int l) {
   return L;
 }
 
+// device copy of a level's cell matrices, referred to by its descriptor
+template <typename T>
+void attach_cell_matrices(LevelDesc &L, DBuf<T> &buf) {
+  if (!march_level(L)) return;
+  const std::vector<T> v = march_tables<T>(L);
+  buf.alloc((long long)v.size());
+  MFS_HIP(hipMemcpy(buf.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+  L.kmat = buf.p;
+  L.kmat_size = (int)sizeof(T);
+}
+
 int n_qp(const mfs_box &b) {
   const int q = b.degree + 1;
   return b.dim == 3 ? q * q * q : q * q;
@@ -163,6 +174,7 @@ struct GMGLevel {
   LevelDesc L;
   long long nu = 0, np = 0;
   DBuf<T> eta, dinvA, dinvS;
+  DBuf<T> kmat;   // cell matrices of a degree-2 level (LevelDesc::kmat)
   DBuf<T> ietan;  // 1 / cellwise viscosity in natural cell order (Schur level operator), set by build()
   DBuf<T> ux, ub, ur, ud, px, pb, pr, pd;
   ChebInfo chA, chS;
@@ -185,8 +197,15 @@ struct GMG {
   // eight tile colours: on coarse levels a colour launch is bound by the latency
   // of one tile, and on the fine level the work-array traffic costs less than
   // the colour tails and the in-kernel gather
+  // (levels with viscosities at the quadrature points, and in-place calls;
+  // set_eta_q1 allocates it before a V-cycle is captured)
   DBuf<T> swork;
-  T *split_for(int) { return swork.p; }
+  T *split_for(int l) {
+    const LevelDesc &L = lv[l]->L;
+    if (laplace || split_work_size(L) == 0) return nullptr;
+    if (swork.n < split_work_size(L)) swork.alloc(split_work_size(lv[top]->L));
+    return swork.p;
+  }
   bool ietan_ok = false;  // GMGLevel::ietan matches the current level viscosity
   // vector Laplace hierarchy of the mesh-deformation solve (kind 0 only): the
   // level operator is the Laplace operator, its diagonal the Laplace diagonal,
@@ -223,6 +242,7 @@ struct GMG {
     for (int l = 0; l < b.n_levels; ++l) {
       auto g = std::make_unique<GMGLevel<T>>();
       g->L = make_level_desc(b, l);
+      if (!laplace) attach_cell_matrices<T>(g->L, g->kmat);
       g->nu = (long long)b.dim * g->L.vnodes;
       g->np = g->L.pnodes;
       g->eta.alloc(g->L.ntiles_total * ct);
@@ -239,10 +259,7 @@ struct GMG {
     }
     top = b.n_levels - 1;
     if (top > 0) xwork.alloc(transfer_work_size(lv[top - 1]->L, lv[top]->L));
-    long long sw = 0;
-    for (auto &g : lv)
-      sw = std::max(sw, split_work_size(g->L));
-    if (sw > 0 && !laplace) swork.alloc(sw);
+    swork.release();
   }
 
   int eta_pq = 0;  // level tables per quadrature point (DGQ1) or per cell (DGQ0)
@@ -272,6 +289,7 @@ struct GMG {
     q1_src = &coef;
     q1_lo = lo;
     q1_hi = hi;
+    (void)split_for(top);
     for (int l = 0; l <= top; ++l) {
       GMGLevel<T> &g = *lv[l];
       const long long na = g.L.ntiles_total * cells_per_tile_of(g.L) * qp_per_cell_of(g.L);
@@ -283,7 +301,12 @@ struct GMG {
     }
   }
 
-  void applyA(int l, Mode mode, const T *x, const T *rhs, T *dst) { applyA_work(l, mode, x, rhs, dst, split_for(l)); }
+  void applyA(int l, Mode mode, const T *x, const T *rhs, T *dst) {
+    GMGLevel<T> &g = *lv[l];
+    if (!laplace && launch_march<T>(OP_ABLOCK, mode, g.L, x, nullptr, g.eta.p, eta_pq, rhs, nullptr, dst, nullptr, st))
+      return;
+    applyA_work(l, mode, x, rhs, dst, split_for(l));
+  }
   // the same apply with the split path's per-cell work array supplied by the caller
   void applyA_work(int l, Mode mode, const T *x, const T *rhs, T *dst, T *work) {
     GMGLevel<T> &g = *lv[l];
@@ -338,6 +361,22 @@ struct GMG {
     return 0.5 * (lo + hi);
   }
 
+  // Level 0 takes up to 100 CG iterations, whose smallest Lanczos value depends
+  // on rounding where the level is ill-conditioned (by up to 1e-4 relative under
+  // 1e-15 perturbations): it keeps the quadrature form of the A block, so that
+  // the coarse smoother does not depend on which kernel the solve runs
+  void apply_estimate(int kind, int l, const T *x, T *dst) {
+    GMGLevel<T> &g = *lv[l];
+    if (kind != 0 || laplace || l > 0) {
+      apply(kind, l, MODE_SET, x, nullptr, dst);
+      return;
+    }
+    LevelDesc L = g.L;
+    L.kmat = nullptr;
+    launch_cell_op<T>(OP_ABLOCK, MODE_SET, L, x, nullptr, g.eta.p, eta_pq, nullptr, nullptr, dst, nullptr, st,
+                      split_for(l));
+  }
+
   void estimate(int kind, int l, ChebInfo &ch, int max_its, double range) {
     GMGLevel<T> &g = *lv[l];
     const long long n = kind == 0 ? g.nu : g.np;
@@ -358,7 +397,7 @@ struct GMG {
       v_cheb_first<T>(dinv, r, z, p, (T)1, true, n, st);  // z = p = D^{-1} r
       double rz = dot(r, z, n);
       for (int it = 1; it <= max_its; ++it) {
-        apply(kind, l, MODE_SET, p, nullptr, q);
+        apply_estimate(kind, l, p, q);
         const double alpha = rz / dot(p, q, n);
         v_axpby<T>((T)(-alpha), q, (T)1, r, n, st);
         alphas.push_back(alpha);
@@ -476,9 +515,8 @@ struct GMG {
     sh->lv.resize(1);
     sh->top = 0;
     sh->xwork.release();
-    const LevelDesc &L0 = sh->lv[0]->L;
     sh->swork.release();
-    if (split_work_size(L0) > 0) sh->swork.alloc(split_work_size(L0));
+    if (eta_pq) (void)sh->split_for(0);
     shadow = std::move(sh);
   }
 
@@ -506,6 +544,7 @@ struct GMG {
       smooth_schur_fused(g, ch, x, b, x_zero, steps);
       return;
     }
+    if (kind == 0 && !laplace && smooth_march(g, ch, x, b, x_zero, steps)) return;
     // residual + update in one pass where the A-block apply is split
     auto fused = [&](T f1, T f2, int first) {
       return kind == 0 && !laplace &&
@@ -534,6 +573,40 @@ struct GMG {
         rho_old = rho;
       }
     }
+  }
+
+  // A-block smoother with the residual fused into every Chebyshev step
+  // (launch_march_cheb), alternating between x and the level's residual buffer
+  // as smooth_schur_fused does; false where the level does not take that kernel
+  bool smooth_march(GMGLevel<T> &g, const ChebInfo &ch, T *x, const T *b, bool x_zero, int steps) {
+    const bool inner = ch.degree >= 2 && std::fabs(ch.delta) >= 1e-40;
+    int swaps = 0;
+    for (int s = 0; s < steps; ++s) swaps += (x_zero && s == 0 ? 0 : 1) + (inner ? ch.degree - 1 : 0);
+    T *cur = x, *alt = g.ur.p;
+    if (x_zero && (swaps & 1)) std::swap(cur, alt);
+    auto step = [&](T f1, T f2, int first) {
+      if (!launch_march_cheb<T>(g.L, cur, b, g.eta.p, eta_pq, g.dinvA.p, g.ud.p, alt, f1, f2, first, st)) return false;
+      std::swap(cur, alt);
+      return true;
+    };
+    const T inv_theta = (T)(1.0 / ch.theta);
+    if (!march_fits<T>(g.L, eta_pq)) return false;
+    for (int s = 0; s < steps; ++s) {
+      if (x_zero && s == 0)
+        v_cheb_first<T>(g.dinvA.p, b, g.ud.p, cur, inv_theta, true, g.nu, st);
+      else
+        step((T)0, inv_theta, 1);
+      if (!inner) continue;
+      const double sigma = ch.theta / ch.delta;
+      double rho_old = ch.delta / ch.theta;
+      for (int k = 1; k < ch.degree; ++k) {
+        const double rho = 1.0 / (2.0 * sigma - rho_old);
+        step((T)(rho * rho_old), (T)(2.0 * rho / ch.delta), 0);
+        rho_old = rho;
+      }
+    }
+    if (cur != x) MFS_HIP(hipMemcpyAsync(x, cur, g.nu * sizeof(T), hipMemcpyDeviceToDevice, st));
+    return true;
   }
 
   // Schur smoother with the residual fused into every Chebyshev step
@@ -690,6 +763,7 @@ struct mfs_handle {
   std::vector<DBuf<double>> geo_lv;
   // work array of the split FP64 Stokes apply on the active level (3D degree 2)
   DBuf<double> swork_stokes;
+  DBuf<double> kmat_top;  // the active level's cell matrices
 
   ~mfs_handle() {
     for (double *p : vchunks) (void)hipFree(p);
@@ -721,8 +795,9 @@ struct mfs_handle {
   // ---- active-level FP64 operators
   // 3D degree 2 on the box: the Stokes apply runs split (one plane-kernel
   // launch over all tiles, then node-wise sums) with this work array
-  double *stokes_work() {
+  double *stokes_work(const double *x, const double *dst) {
     const LevelDesc &T = Ltop();
+    if (march_fits<double>(T, active_per_qp) && !(x < dst + n && dst < x + n)) return nullptr;
     if (T.dim != 3 || T.k != 2 || T.geo) return nullptr;
     const long long n = stokes_split_work_size(T);
     if (swork_stokes.n != n) swork_stokes.alloc(n);
@@ -730,7 +805,7 @@ struct mfs_handle {
   }
   void stokes(Mode mode, const double *x, const double *rhs, double *dst) {
     launch_cell_op<double>(OP_STOKES, mode, Ltop(), x, x + nu, eta_active.p, active_per_qp, rhs,
-                           rhs ? rhs + nu : nullptr, dst, dst + nu, st, stokes_work());
+                           rhs ? rhs + nu : nullptr, dst, dst + nu, st, stokes_work(x, dst));
     if (fs_on) launch_free_surface(Ltop(), fs_faces, fs_stab.p, x, fs_sv.p, mode == MODE_RESID ? -1.0 : 1.0, dst, st);
   }
   void ablock_active(Mode mode, const double *x, const double *rhs, double *dst) {
@@ -1472,6 +1547,7 @@ void create(const mfs_box *b, int prec, mfs_handle **out) {
   MFS_HIP(hipStreamCreateWithFlags(&h->st, hipStreamNonBlocking));
   for (int l = 0; l < b->n_levels; ++l) h->L.push_back(make_level_desc(h->box, l));
   h->top = b->n_levels - 1;
+  attach_cell_matrices<double>(h->L[h->top], h->kmat_top);
   h->nu = (long long)b->dim * h->Ltop().vnodes;
   h->np = h->Ltop().pnodes;
   h->n = h->nu + h->np;

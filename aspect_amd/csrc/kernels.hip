@@ -1460,6 +1460,7 @@ void launch_cell_op(Op op, Mode mode, const LevelDesc &L, const T *src_u, const 
                     int eta_per_qp, const T *rhs_u, const T *rhs_p, T *dst_u, T *dst_p, hipStream_t st,
                     T *split_work) {
   check_op_args(op, mode, src_u, src_p, eta, rhs_u, rhs_p, dst_u, dst_p);
+  if (launch_march<T>(op, mode, L, src_u, src_p, eta, eta_per_qp, rhs_u, rhs_p, dst_u, dst_p, st)) return;
   if (launch_cell_q2<T>(op, mode, L, src_u, src_p, eta, eta_per_qp, rhs_u, rhs_p, dst_u, dst_p, st, split_work))
     return;
   if (op == OP_ABLOCK && split_work && L.dim == 2 && L.k == 2 && !L.geo) {

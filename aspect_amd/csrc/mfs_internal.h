@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 namespace mfs {
 
@@ -59,6 +60,14 @@ struct ChebArgs {
   T f1, f2;
   int first;
 };
+// The same step where x goes to another buffer (the kernel's source and destination)
+template <typename T>
+struct ChebOut {
+  const T *dinv;
+  T *d;
+  T f1, f2;
+  int first;
+};
 
 // Geometry of one uniform box level.  Velocity nodes: (k*n+1) per direction,
 // pressure nodes ((k-1)*n+1); both lexicographic with x fastest; the velocity
@@ -90,6 +99,10 @@ struct LevelDesc {
   // pressure (a lexicographic in the cell, x fastest)
   const int *cell_u;
   const int *cell_p;
+  // cell matrices of a uniform degree-2 level (march_tables) on the device, in
+  // elements of kmat_size bytes; nullptr: none
+  const void *kmat;
+  int kmat_size;
 };
 
 // Mesh constants of a level in the arithmetic type of a kernel (kernel
@@ -180,6 +193,24 @@ bool launch_cell_planes(Op op, Mode mode, const LevelDesc &L, const T *src_u, co
 template <typename T>
 bool launch_ablock_cheb(const LevelDesc &L, T *x, const T *b, const T *eta, int eta_per_qp, const T *dinv, T *d,
                         T f1, T f2, int first, T *split_work, hipStream_t st);
+
+// Degree-2 box levels with one viscosity per cell (kernels_march.hip): Stokes
+// (FP64) and A-block applies in one launch from the level's cell matrices, and
+// the A-block residual fused with a Jacobi-Chebyshev step, x_out = x_in + d
+// (x_out != x_in).  false (nothing launched) where the level, the viscosity
+// table or an in-place call does not fit; march_tables: the table behind
+// LevelDesc::kmat.
+bool march_level(const LevelDesc &L);
+template <typename T>
+bool march_fits(const LevelDesc &L, int eta_per_qp);
+template <typename T>
+std::vector<T> march_tables(const LevelDesc &L);
+template <typename T>
+bool launch_march(Op op, Mode mode, const LevelDesc &L, const T *src_u, const T *src_p, const T *eta, int eta_per_qp,
+                  const T *rhs_u, const T *rhs_p, T *dst_u, T *dst_p, hipStream_t st);
+template <typename T>
+bool launch_march_cheb(const LevelDesc &L, const T *x_in, const T *b, const T *eta, int eta_per_qp, const T *dinv, T *d,
+                       T *x_out, T f1, T f2, int first, hipStream_t st);
 
 // Transfers between level Lc (coarse) and Lf = refined Lc.  kind 0 velocity, 1 pressure.
 // work: nullptr, or transfer_work_size(Lc, Lf) elements for the separable

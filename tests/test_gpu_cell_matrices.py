@@ -1,0 +1,82 @@
+"""Applies from the cell matrices (levels with one viscosity per cell) at the
+edges of their boxes of columns and marches, against the quadrature form: an
+in-place call cannot take the one-launch kernel (a workgroup would overwrite
+what its neighbours read) and runs the split quadrature kernels."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from aspect_amd import StokesMatrixFreeHandler, make_box
+
+pytestmark = pytest.mark.gpu
+
+MIXED = (1, 2, 0, 1, 1, 2)
+# a box owns 7 x 7 columns of cells or a longer strip, a march 1 to 11 layers:
+# one cell, one short of / exactly / one past a box, strips, several marches
+SIZES = [(1, 1, 1), (6, 7, 8), (7, 8, 2), (8, 6, 13), (21, 2, 3), (2, 30, 5), (15, 14, 12), (40, 33, 24)]
+# a row sums at most 8 cells x 36 products after 6 sums: ~ sqrt(8 * 42) rounding errors of the largest
+# terms, which the smooth part of a random field leaves ~ 10 times larger than the row
+TOL = {"fp64": 200 * 2.0 ** -53 * 10, "fp32": 200 * 2.0 ** -24 * 10}
+
+
+def _box(n, bc, compressible, prec):
+    h = StokesMatrixFreeHandler(make_box(len(n), 2, n, 1, (1.0, 0.7, 1.9), bc, compressible, 1.3), prec)
+    s = h.sizes(0)
+    rng = np.random.default_rng(sum(n))
+    h.assemble(np.exp(rng.normal(scale=2.0, size=(s["cells"], h.n_qp))), "harmonic")
+    return h, s, rng
+
+
+def _against_in_place(apply, x):
+    y, z = torch.full_like(x, float("nan")), x.clone()
+    torch.cuda.synchronize()
+    apply(x.data_ptr(), y.data_ptr())
+    apply(z.data_ptr(), z.data_ptr())
+    torch.cuda.synchronize()
+    return float((y - z).norm() / z.norm())
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("compressible", [False, True])
+@pytest.mark.parametrize("n", SIZES + [(1, 1), (7, 7), (8, 6), (50, 3), (33, 40)])
+def test_ablock_apply_matches_quadrature(n, compressible, prec):
+    h, s, rng = _box(n, MIXED, compressible, prec)
+    print("ablock", n, prec, compressible, flush=True)
+    x = torch.tensor(rng.normal(size=s["nu"]), dtype=torch.float64 if prec == "fp64" else torch.float32, device="cuda:0")
+    assert _against_in_place(lambda a, b: h.ablock_vmult_device(0, a, b), x) < TOL[prec]
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_stokes_apply_matches_quadrature(n):
+    for bc in (MIXED, (2,) * 6, (0,) * 6):
+        h, s, rng = _box(n, bc, False, "fp64")
+        print("stokes", n, bc, flush=True)
+        x = torch.tensor(rng.normal(size=s["nu"] + s["np"]), device="cuda:0")
+        assert _against_in_place(h.stokes_vmult_device, x) < TOL["fp64"]
+
+
+@pytest.mark.parametrize("n", [(1, 1), (7, 7), (8, 6), (50, 3)])
+def test_stokes_2d_matches_oracle(n):
+    # the 2D quadrature form runs in tile colours and takes no in-place call
+    bc = MIXED[:4]
+    h, s, rng = _box(n, bc, True, "fp64")
+    eta = np.exp(np.random.default_rng(sum(n)).normal(scale=2.0, size=(s["cells"], 9)))
+    p = O.make_problem(2, 2, n, 1, (1.0, 0.7), bc, pressure_scaling=1.3, compressible=True)
+    x = rng.normal(size=s["nu"] + s["np"])
+    ref = O.stokes_vmult(p, 0, 1.0 / np.mean(1.0 / eta, axis=1), x)
+    assert np.linalg.norm(h.stokes_vmult(x) - ref) < TOL["fp64"] * np.linalg.norm(ref)
+
+
+def test_source_outside_the_mesh_is_not_read_into_rows():
+    # columns beyond the mesh read the nearest cells and discard the values:
+    # an infinity at one node reaches only the rows of the cells that hold it
+    h, s, rng = _box((9, 8, 10), (0,) * 6, False, "fp64")
+    x = torch.tensor(rng.normal(size=s["nu"]), device="cuda:0")
+    x[0] = float("inf")
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    h.ablock_vmult_device(0, x.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    bad = ~torch.isfinite(y.cpu().reshape(3, 21, 17, 19))
+    assert bad[:, :3, :3, :3].any() and not bad[:, 3:].any() and not bad[:, :, 3:].any() and not bad[..., 3:].any()
