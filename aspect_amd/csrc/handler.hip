@@ -191,7 +191,6 @@ struct GMG {
   // whenever those change
   bool graphs = true;
   hipGraphExec_t vexec[2] = {nullptr, nullptr};
-  DBuf<T> xwork;  // work arrays of the separable transfers (sized for the finest pair)
   // A-block applies in the V-cycle run as two launches over all tiles through
   // this work array (per-cell contributions, then node-wise sums) instead of
   // eight tile colours: on coarse levels a colour launch is bound by the latency
@@ -258,7 +257,6 @@ struct GMG {
       lv.push_back(std::move(g));
     }
     top = b.n_levels - 1;
-    if (top > 0) xwork.alloc(transfer_work_size(lv[top - 1]->L, lv[top]->L));
     swork.release();
   }
 
@@ -514,7 +512,6 @@ struct GMG {
     MFS_HIP(hipStreamSynchronize(st));
     sh->lv.resize(1);
     sh->top = 0;
-    sh->xwork.release();
     sh->swork.release();
     if (eta_pq) (void)sh->split_for(0);
     shadow = std::move(sh);
@@ -687,9 +684,9 @@ struct GMG {
     smooth(kind, l, x, b, true, steps);
     apply(kind, l, MODE_RESID, x, b, r);
     GMGLevel<T> &c = *lv[l - 1];
-    launch_restrict<T>(kind, c.L, g.L, r, kind == 0 ? c.ub.p : c.pb.p, st, xwork.p);
+    launch_restrict<T>(kind, c.L, g.L, r, kind == 0 ? c.ub.p : c.pb.p, st);
     vcycle_level(kind, l - 1);
-    launch_prolongate<T>(kind, c.L, g.L, kind == 0 ? c.ux.p : c.px.p, x, true, st, xwork.p);
+    launch_prolongate<T>(kind, c.L, g.L, kind == 0 ? c.ux.p : c.px.p, x, true, st);
     smooth(kind, l, x, b, false, steps);
   }
 
@@ -2286,9 +2283,7 @@ int mfs_prolongate(mfs_handle *h, int fine_level, int kind, const double *src, d
     const long long nf = kind == 0 ? (long long)h->box.dim * Lf.vnodes : Lf.pnodes;
     HostIO io{h};
     io.in(h->w1.p, src, nc);
-    DBuf<double> work;
-    work.alloc(transfer_work_size(Lc, Lf));
-    launch_prolongate<double>(kind, Lc, Lf, h->w1.p, h->w2.p, false, h->st, work.p);
+    launch_prolongate<double>(kind, Lc, Lf, h->w1.p, h->w2.p, false, h->st);
     io.out(dst, h->w2.p, nf);
     return MFS_OK;
   });
@@ -2304,9 +2299,7 @@ int mfs_restrict(mfs_handle *h, int fine_level, int kind, const double *src, dou
     const long long nf = kind == 0 ? (long long)h->box.dim * Lf.vnodes : Lf.pnodes;
     HostIO io{h};
     io.in(h->w1.p, src, nf);
-    DBuf<double> work;
-    work.alloc(transfer_work_size(Lc, Lf));
-    launch_restrict<double>(kind, Lc, Lf, h->w1.p, h->w2.p, h->st, work.p);
+    launch_restrict<double>(kind, Lc, Lf, h->w1.p, h->w2.p, h->st);
     io.out(dst, h->w2.p, nc);
     return MFS_OK;
   });

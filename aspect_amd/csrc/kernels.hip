@@ -1733,249 +1733,222 @@ __global__ void k_restrict(const LevelDesc Lc, const LevelDesc Lf, const int kin
   }
 }
 
-// 3D transfers with fixed tap patterns for Q2 velocity (KK = 2, nodes 0, 1/2, 1)
-// and Q1 pressure (KK = 1).  Prolongation row of fine local node r in its
-// coarse cell: the Lagrange basis at r / (2 KK); the zero taps are skipped at
-// compile time.
+// Degree-2 transfers (Q2 velocity KK = 2, Q1 pressure KK = 1), each in one
+// launch: a thread takes the nodes that a coarse cell owns in one plane z (the
+// plane's taps are uniform over the block) and contracts x and y in registers,
+// so neither direction goes through memory.  Bound by the launch and one chain of
+// loads: on the levels of 32^3 and below in double 8.1 us for the velocity and
+// 4.2 us for the pressure, where one pass per direction with two work arrays took
+// 13 us (three launches of 4.3 us); 64^3 and below in single 12.8 us (18.3 us).
+// Prolongation: fine local node r of a coarse cell is the Lagrange basis at
+// r / (2 KK); compile-time rows, so zero taps vanish.  Restriction, its
+// transpose: a coarse vertex takes the fine nodes at distance 0 (1), 1 (3/8) and
+// 3 (-1/8) for KK = 2, 0 (1) and 1 (1/2) for KK = 1; a coarse midpoint 0 (1) and 1
+// (3/4).  Constrained DoFs read as zero and written as zero on both levels.
 template <int KK>
-struct ProlongTaps;
-template <>
-struct ProlongTaps<2> {
-  static constexpr double W[5][3] = {
+constexpr __host__ __device__ double prolong_tap(int r, int m) {
+  constexpr double W2[5][3] = {
       {1.0, 0.0, 0.0}, {0.375, 0.75, -0.125}, {0.0, 1.0, 0.0}, {-0.125, 0.75, 0.375}, {0.0, 0.0, 1.0}};
-};
-template <>
-struct ProlongTaps<1> {
-  static constexpr double W[3][2] = {{1.0, 0.0}, {0.5, 0.5}, {0.0, 1.0}};
-};
-
-__device__ __forceinline__ bool con_node(const LevelDesc &L, int comp, int gx, int gy, int gz) {
-  const int g[3] = {gx, gy, gz};
-  bool con = false;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int b = g[d] == 0 ? L.bc[2 * d] : (g[d] == L.nv[d] - 1 ? L.bc[2 * d + 1] : 0);
-    con = con || b == 2 || (b == 1 && comp == d);
-  }
-  return con;
+  constexpr double W1[3][2] = {{1.0, 0.0}, {0.5, 0.5}, {0.0, 1.0}};
+  return KK == 2 ? W2[r][m] : W1[r < 3 ? r : 2][m < 2 ? m : 1];
 }
-
-// Separable transfers (degree 2): the tensor-product prolongation P = Px Py Pz
-// (and R = P^T) applied one direction per pass through two work arrays (2D:
-// Px Py, one work array).  Each pass
-// is a 1D stencil along one axis of an (n0, n1, n2) array per component:
-// restriction, coarse node m takes the fine nodes 2m + o (a coarse vertex: o = 0
-// (1), +-1 (3/8), +-3 (-1/8) for KK = 2, o = 0 (1), +-1 (1/2) for KK = 1; a cell
-// midpoint node: o = 0 (1), +-1 (3/4)), prolongation, fine node g takes its coarse cell's nodes with
-// the row of ProlongTaps.  Constrained DoFs: the first restriction pass reads
-// constrained fine nodes as zero and the last one zeroes constrained coarse
-// nodes; the first prolongation pass reads constrained coarse nodes as zero
-// and the last one zeroes constrained fine nodes.
-struct Dims3 {
-  int n[3];
-};
-// Grid of the passes: x over the nodes of an xy plane of the output, y over
-// (z, comp); 32-bit offsets (the launcher checks the sizes).  Arithmetic in T.
-template <int KK, typename T>
-__global__ void k_restrict_pass(const LevelDesc Lc, const LevelDesc Lf, const int ax, const Dims3 din, const Dims3 dout,
-                                const int ncomp, const int first, const int last, const T *__restrict__ in,
-                                T *__restrict__ out) {
-  const unsigned plane = (unsigned)(dout.n[0] * dout.n[1]);
-  const unsigned pidx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pidx >= plane) return;
-  const int row = blockIdx.y;  // z + nz * comp
-  const int comp = row / dout.n[2];
-  const int o1 = (int)(pidx / (unsigned)dout.n[0]);
-  const int o[3] = {(int)pidx - o1 * dout.n[0], o1, row - comp * dout.n[2]};
-  const int stride = ax == 0 ? 1 : (ax == 1 ? din.n[0] : din.n[0] * din.n[1]);
-  const int m = o[ax];
-  int base[3] = {o[0], o[1], o[2]};
-  base[ax] = 0;
-  const int b0 = comp * din.n[0] * din.n[1] * din.n[2] + base[0] + din.n[0] * (base[1] + din.n[1] * base[2]);
-  constexpr bool VEL = KK == 2;
-  constexpr int NO = VEL ? 5 : 3;
-  const bool vertex = !VEL || (m & 1) == 0;
-  T acc = 0;
-#pragma unroll
-  for (int k = 0; k < NO; ++k) {
-    int off;
-    T wv;
-    if constexpr (VEL) {
-      off = k == 0 ? -3 : (k == 1 ? -1 : (k == 2 ? 0 : (k == 3 ? 1 : 3)));
-      wv = vertex ? (k == 2 ? T(1) : (k == 1 || k == 3 ? T(0.375) : T(-0.125)))
-                  : (k == 2 ? T(1) : (k == 1 || k == 3 ? T(0.75) : T(0)));
-    } else {
-      off = k - 1;
-      wv = k == 1 ? T(1) : T(0.5);
-    }
-    const int g = 2 * m + off;
-    bool ok = wv != T(0) && g >= 0 && g < din.n[ax];
-    if (VEL && first) {
-      int f[3] = {o[0], o[1], o[2]};
-      f[ax] = g;
-      ok = ok && !con_node(Lf, comp, f[0], f[1], f[2]);
-    }
-    const T v = in[ok ? b0 + g * stride : b0];
-    acc += ok ? wv * v : T(0);
-  }
-  if (last && VEL && con_node(Lc, comp, o[0], o[1], o[2])) acc = 0;
-  out[(long long)row * plane + pidx] = acc;
+// restriction of the fine node at offset o from 2 KK e to local node i (0 vertex, 1 midpoint) of coarse cell e
+template <int KK>
+constexpr __host__ __device__ double restrict_tap(int i, int o) {
+  const int t = KK == 2 ? (o < 2 * i ? 2 * i - o : o - 2 * i) : (o < 0 ? -o : o);
+  if (KK == 1) return t == 0 ? 1.0 : (t == 1 ? 0.5 : 0.0);
+  if (i == 0) return t == 0 ? 1.0 : (t == 1 ? 0.375 : (t == 3 ? -0.125 : 0.0));
+  return t == 0 ? 1.0 : (t == 1 ? 0.75 : 0.0);
 }
-template <int KK, typename T>
-__global__ void k_prolong_pass(const LevelDesc Lc, const LevelDesc Lf, const int ax, const Dims3 din, const Dims3 dout,
-                               const int ncomp, const int first, const int last, const int add,
-                               const T *__restrict__ in, T *__restrict__ out) {
-  const unsigned plane = (unsigned)(dout.n[0] * dout.n[1]);
-  const unsigned pidx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pidx >= plane) return;
-  const int row = blockIdx.y;  // z + nz * comp
-  const int comp = row / dout.n[2];
-  const int o1 = (int)(pidx / (unsigned)dout.n[0]);
-  const int o[3] = {(int)pidx - o1 * dout.n[0], o1, row - comp * dout.n[2]};
-  const int stride = ax == 0 ? 1 : (ax == 1 ? din.n[0] : din.n[0] * din.n[1]);
-  const int g = o[ax];
-  const int ncell = Lc.n[ax];
-  int e = g / (2 * KK), rr = g - 2 * KK * e;
-  if (e == ncell) {
-    e = ncell - 1;
-    rr = 2 * KK;
-  }
-  int base[3] = {o[0], o[1], o[2]};
-  base[ax] = 0;
-  const int b0 = comp * din.n[0] * din.n[1] * din.n[2] + base[0] + din.n[0] * (base[1] + din.n[1] * base[2]);
+// is node g of a direction constrained for component comp (faces lo and hi)?
+__device__ __forceinline__ bool face_fixed(int g, int last, int lo, int hi, bool normal) {
+  const int b = g == 0 ? lo : (g == last ? hi : 0);
+  return b == 2 || (b == 1 && normal);
+}
+// grid: x over the coarse cells of a plane (one more per direction: the last
+// nodes), y over (component, plane of the output); 32-bit offsets
+template <int DIM, int KK, typename T>
+__global__ void __launch_bounds__(128) k_prolong_cells(const LevelDesc Lc, const LevelDesc Lf, const int add,
+                                                       const T *__restrict__ src, T *__restrict__ dst) {
   constexpr bool VEL = KK == 2;
-  T acc = 0;
+  const int *nc = VEL ? Lc.nv : Lc.np, *nf = VEL ? Lf.nv : Lf.np;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ey = i / (Lc.n[0] + 1), ex = i - ey * (Lc.n[0] + 1);
+  if (ey > Lc.n[1]) return;
+  const int comp = blockIdx.y / (DIM == 3 ? nf[2] : 1), gz = blockIdx.y - comp * (DIM == 3 ? nf[2] : 1);
+  bool okx[KK + 1], oky[KK + 1];
+  int ox[KK + 1], oy[KK + 1];
 #pragma unroll
-  for (int mm = 0; mm <= KK; ++mm) {
-    T wv = (T)ProlongTaps<KK>::W[0][mm];
-#pragma unroll
-    for (int q = 1; q <= 2 * KK; ++q) wv = rr == q ? (T)ProlongTaps<KK>::W[q][mm] : wv;
-    const int cidx = KK * e + mm;
-    bool ok = wv != T(0);
-    if (VEL && first) {
-      int c[3] = {o[0], o[1], o[2]};
-      c[ax] = cidx;
-      ok = ok && !con_node(Lc, comp, c[0], c[1], c[2]);
-    }
-    const T v = in[b0 + cidx * stride];
-    acc += ok ? wv * v : T(0);
+  for (int m = 0; m <= KK; ++m) {
+    const int x = KK * ex + m, y = KK * ey + m;
+    ox[m] = min(x, nc[0] - 1);
+    oy[m] = min(y, nc[1] - 1) * nc[0];
+    okx[m] = !VEL || !face_fixed(x, nc[0] - 1, Lc.bc[0], Lc.bc[1], comp == 0);
+    oky[m] = !VEL || !face_fixed(y, nc[1] - 1, Lc.bc[2], Lc.bc[3], comp == 1);
   }
-  if (last && VEL && con_node(Lf, comp, o[0], o[1], o[2])) acc = 0;
-  const long long oi = (long long)row * plane + pidx;
-  out[oi] = add ? (T)(out[oi] + acc) : acc;
+  T u[KK + 1][KK + 1];
+#pragma unroll
+  for (int a = 0; a <= KK; ++a)
+#pragma unroll
+    for (int m = 0; m <= KK; ++m) u[a][m] = 0;
+  const T *const base = src + comp * (nc[0] * nc[1] * (DIM == 3 ? nc[2] : 1));
+  const int ez = gz / (2 * KK), rz = gz - 2 * KK * ez;
+#pragma unroll
+  for (int t = 0; t < (DIM == 3 ? KK + 1 : 1); ++t) {
+    T w = 1;
+    int z = 0;
+    if constexpr (DIM == 3) {
+      w = 0;
+#pragma unroll
+      for (int r = 0; r < 2 * KK; ++r) w = rz == r ? (T)prolong_tap<KK>(r, t) : w;
+      z = KK * ez + t;
+      if (w == T(0) || (VEL && face_fixed(z, nc[2] - 1, Lc.bc[4], Lc.bc[5], comp == 2))) continue;  // uniform
+    }
+    const T *const p = base + z * (nc[0] * nc[1]);
+#pragma unroll
+    for (int a = 0; a <= KK; ++a)
+#pragma unroll
+      for (int m = 0; m <= KK; ++m) {
+        const T v = p[oy[a] + ox[m]];
+        u[a][m] += okx[m] && oky[a] ? w * v : (T)0;
+      }
+  }
+  const bool fz = DIM == 3 && VEL && face_fixed(gz, nf[2] - 1, Lf.bc[4], Lf.bc[5], comp == 2);
+#pragma unroll
+  for (int ry = 0; ry < 2 * KK; ++ry) {
+    const int gy = 2 * KK * ey + ry;
+    if (gy >= nf[1]) break;
+    T line[KK + 1];
+#pragma unroll
+    for (int m = 0; m <= KK; ++m) {
+      line[m] = 0;
+#pragma unroll
+      for (int a = 0; a <= KK; ++a)
+        if (prolong_tap<KK>(ry, a) != 0.0) line[m] += (T)prolong_tap<KK>(ry, a) * u[a][m];
+    }
+    const bool fy = fz || (VEL && face_fixed(gy, nf[1] - 1, Lf.bc[2], Lf.bc[3], comp == 1));
+    T *const out = dst + ((comp * (DIM == 3 ? nf[2] : 1) + gz) * nf[1] + gy) * nf[0];
+#pragma unroll
+    for (int rx = 0; rx < 2 * KK; ++rx) {
+      const int gx = 2 * KK * ex + rx;
+      if (gx >= nf[0]) break;
+      T v = 0;
+#pragma unroll
+      for (int m = 0; m <= KK; ++m)
+        if (prolong_tap<KK>(rx, m) != 0.0) v += (T)prolong_tap<KK>(rx, m) * line[m];
+      if (fy || (VEL && face_fixed(gx, nf[0] - 1, Lf.bc[0], Lf.bc[1], comp == 0))) v = 0;
+      out[gx] = add ? out[gx] + v : v;
+    }
+  }
+}
+template <int DIM, int KK, typename T>
+__global__ void __launch_bounds__(128) k_restrict_cells(const LevelDesc Lc, const LevelDesc Lf,
+                                                        const T *__restrict__ src, T *__restrict__ dst) {
+  constexpr bool VEL = KK == 2;
+  constexpr int LO = VEL ? -3 : -1, NO = VEL ? 7 : 3;  // fine offsets LO .. LO + NO - 1 around 2 KK e
+  const int *nc = VEL ? Lc.nv : Lc.np, *nf = VEL ? Lf.nv : Lf.np;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ey = i / (Lc.n[0] + 1), ex = i - ey * (Lc.n[0] + 1);
+  if (ey > Lc.n[1]) return;
+  const int comp = blockIdx.y / (DIM == 3 ? nc[2] : 1), mz = blockIdx.y - comp * (DIM == 3 ? nc[2] : 1);
+  bool okx[NO];
+  int ox[NO];
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    const int g = 2 * KK * ex + LO + o;
+    ox[o] = min(max(g, 0), nf[0] - 1);
+    okx[o] = g >= 0 && g < nf[0] && !(VEL && face_fixed(g, nf[0] - 1, Lf.bc[0], Lf.bc[1], comp == 0));
+  }
+  T acc[KK][KK];
+#pragma unroll
+  for (int j = 0; j < KK; ++j)
+#pragma unroll
+    for (int k = 0; k < KK; ++k) acc[j][k] = 0;
+  const T *const base = src + comp * (nf[0] * nf[1] * (DIM == 3 ? nf[2] : 1));
+  const int ez = mz / KK, iz = mz - KK * ez;
+#pragma unroll
+  for (int a = 0; a < (DIM == 3 ? NO : 1); ++a) {
+    T wz = 1;
+    int z = 0;
+    if constexpr (DIM == 3) {
+      wz = iz == 0 ? (T)restrict_tap<KK>(0, LO + a) : (T)restrict_tap<KK>(1, LO + a);
+      z = 2 * KK * ez + LO + a;
+      if (wz == T(0) || z < 0 || z >= nf[2]) continue;  // uniform
+      if (VEL && face_fixed(z, nf[2] - 1, Lf.bc[4], Lf.bc[5], comp == 2)) continue;
+    }
+#pragma unroll
+    for (int b = 0; b < NO; ++b) {
+      if (restrict_tap<KK>(0, LO + b) == 0.0 && (KK == 1 || restrict_tap<KK>(1, LO + b) == 0.0)) continue;
+      const int y = 2 * KK * ey + LO + b;
+      const bool oky = y >= 0 && y < nf[1] && !(VEL && face_fixed(y, nf[1] - 1, Lf.bc[2], Lf.bc[3], comp == 1));
+      const T *const p = base + (z * nf[1] + min(max(y, 0), nf[1] - 1)) * nf[0];
+      T row[KK];
+#pragma unroll
+      for (int k = 0; k < KK; ++k) row[k] = 0;
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        if (restrict_tap<KK>(0, LO + o) == 0.0 && (KK == 1 || restrict_tap<KK>(1, LO + o) == 0.0)) continue;
+        const T r = p[ox[o]], v = okx[o] && oky ? r : (T)0;
+#pragma unroll
+        for (int k = 0; k < KK; ++k)
+          if (restrict_tap<KK>(k, LO + o) != 0.0) row[k] += (T)restrict_tap<KK>(k, LO + o) * v;
+      }
+#pragma unroll
+      for (int j = 0; j < KK; ++j)
+        if (restrict_tap<KK>(j, LO + b) != 0.0)
+#pragma unroll
+          for (int k = 0; k < KK; ++k) acc[j][k] += wz * (T)restrict_tap<KK>(j, LO + b) * row[k];
+    }
+  }
+  const bool fz = DIM == 3 && VEL && face_fixed(mz, nc[2] - 1, Lc.bc[4], Lc.bc[5], comp == 2);
+#pragma unroll
+  for (int j = 0; j < KK; ++j)
+#pragma unroll
+    for (int k = 0; k < KK; ++k) {
+      const int x = KK * ex + k, y = KK * ey + j;
+      if (x >= nc[0] || y >= nc[1]) continue;
+      const bool fixed = fz || (VEL && (face_fixed(x, nc[0] - 1, Lc.bc[0], Lc.bc[1], comp == 0) ||
+                                        face_fixed(y, nc[1] - 1, Lc.bc[2], Lc.bc[3], comp == 1)));
+      dst[((comp * (DIM == 3 ? nc[2] : 1) + mz) * nc[1] + y) * nc[0] + x] = fixed ? (T)0 : acc[j][k];
+    }
 }
 
 template <typename T>
-static void run_sep_transfer(bool prolong, int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src, T *dst,
-                             bool add, T *work, hipStream_t st) {
+static void run_cell_transfer(bool prolong, int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src, T *dst,
+                              bool add, hipStream_t st) {
   const bool vel = kind == 0;
+  const long long nfine = vel ? (long long)Lf.dim * Lf.vnodes : Lf.pnodes;
+  if (nfine >= (1LL << 31)) throw std::runtime_error("level too large for the transfers (32-bit offsets)");
   const int ncomp = vel ? Lf.dim : 1;
-  if (Lf.dim == 2) {  // two passes through one work array (c, f)
-    Dims3 dc, df, d1;
-    for (int d = 0; d < 3; ++d) {
-      dc.n[d] = vel ? Lc.nv[d] : Lc.np[d];
-      df.n[d] = vel ? Lf.nv[d] : Lf.np[d];
-    }
-    if ((long long)df.n[0] * df.n[1] * ncomp >= (1LL << 31))
-      throw std::runtime_error("level too large for the separable transfers (32-bit offsets)");
-    d1 = prolong ? dc : df;
+  const LevelDesc &L = prolong ? Lf : Lc;
+  const int planes = L.dim == 3 ? (vel ? L.nv[2] : L.np[2]) : 1;
+  const dim3 grid((unsigned)(((long long)(Lc.n[0] + 1) * (Lc.n[1] + 1) + 127) / 128), (unsigned)(planes * ncomp));
+  auto go = [&](auto dimc, auto kkc) {
+    constexpr int D = decltype(dimc)::value, KK = decltype(kkc)::value;
     if (prolong)
-      d1.n[1] = df.n[1];  // coarse -> (c, f) -> fine
+      hipLaunchKernelGGL((k_prolong_cells<D, KK, T>), grid, dim3(128), 0, st, Lc, Lf, add ? 1 : 0, src, dst);
     else
-      d1.n[0] = dc.n[0];  // fine -> (c, f) -> coarse
-    auto blocks = [&](const Dims3 &d) {
-      return dim3((unsigned)(((long long)d.n[0] * d.n[1] + 255) / 256), (unsigned)ncomp);
-    };
-    if (!prolong) {
-      if (vel) {
-        hipLaunchKernelGGL((k_restrict_pass<2, T>), blocks(d1), dim3(256), 0, st, Lc, Lf, 0, df, d1, ncomp, 1, 0, src,
-                           work);
-        hipLaunchKernelGGL((k_restrict_pass<2, T>), blocks(dc), dim3(256), 0, st, Lc, Lf, 1, d1, dc, ncomp, 0, 1,
-                           (const T *)work, dst);
-      } else {
-        hipLaunchKernelGGL((k_restrict_pass<1, T>), blocks(d1), dim3(256), 0, st, Lc, Lf, 0, df, d1, ncomp, 0, 0, src,
-                           work);
-        hipLaunchKernelGGL((k_restrict_pass<1, T>), blocks(dc), dim3(256), 0, st, Lc, Lf, 1, d1, dc, ncomp, 0, 0,
-                           (const T *)work, dst);
-      }
-    } else {
-      if (vel) {
-        hipLaunchKernelGGL((k_prolong_pass<2, T>), blocks(d1), dim3(256), 0, st, Lc, Lf, 1, dc, d1, ncomp, 1, 0, 0, src,
-                           work);
-        hipLaunchKernelGGL((k_prolong_pass<2, T>), blocks(df), dim3(256), 0, st, Lc, Lf, 0, d1, df, ncomp, 0, 1,
-                           add ? 1 : 0, (const T *)work, dst);
-      } else {
-        hipLaunchKernelGGL((k_prolong_pass<1, T>), blocks(d1), dim3(256), 0, st, Lc, Lf, 1, dc, d1, ncomp, 0, 0, 0, src,
-                           work);
-        hipLaunchKernelGGL((k_prolong_pass<1, T>), blocks(df), dim3(256), 0, st, Lc, Lf, 0, d1, df, ncomp, 0, 0,
-                           add ? 1 : 0, (const T *)work, dst);
-      }
-    }
-    MFS_HIP(hipGetLastError());
-    return;
-  }
-  Dims3 dc, df;
-  for (int d = 0; d < 3; ++d) {
-    dc.n[d] = vel ? Lc.nv[d] : Lc.np[d];
-    df.n[d] = vel ? Lf.nv[d] : Lf.np[d];
-  }
-  if ((long long)df.n[0] * df.n[1] * df.n[2] * ncomp >= (1LL << 31))
-    throw std::runtime_error("level too large for the separable transfers (32-bit offsets)");
-  auto blocks = [&](const Dims3 &d) {
-    return dim3((unsigned)(((long long)d.n[0] * d.n[1] + 255) / 256), (unsigned)(d.n[2] * ncomp));
+      hipLaunchKernelGGL((k_restrict_cells<D, KK, T>), grid, dim3(128), 0, st, Lc, Lf, src, dst);
   };
-  if (!prolong) {
-    // x, y, z: fine -> (c, f, f) -> (c, c, f) -> coarse
-    Dims3 d1 = df, d2 = df;
-    d1.n[0] = dc.n[0];
-    d2.n[0] = dc.n[0];
-    d2.n[1] = dc.n[1];
-    T *t1 = work, *t2 = work + (long long)d1.n[0] * d1.n[1] * d1.n[2] * ncomp;
-    const T *ins[3] = {src, t1, t2};
-    T *outs[3] = {t1, t2, dst};
-    const Dims3 di[3] = {df, d1, d2}, dd[3] = {d1, d2, dc};
-    for (int ax = 0; ax < 3; ++ax) {
-      if (vel)
-        hipLaunchKernelGGL((k_restrict_pass<2, T>), blocks(dd[ax]), dim3(256), 0, st, Lc, Lf, ax, di[ax], dd[ax],
-                           ncomp, ax == 0 ? 1 : 0, ax == 2 ? 1 : 0, ins[ax], outs[ax]);
-      else
-        hipLaunchKernelGGL((k_restrict_pass<1, T>), blocks(dd[ax]), dim3(256), 0, st, Lc, Lf, ax, di[ax], dd[ax],
-                           ncomp, 0, 0, ins[ax], outs[ax]);
-    }
-  } else {
-    // z, y, x: coarse -> (c, c, f) -> (c, f, f) -> fine
-    Dims3 d1 = dc, d2 = dc;
-    d1.n[2] = df.n[2];
-    d2.n[2] = df.n[2];
-    d2.n[1] = df.n[1];
-    T *t1 = work, *t2 = work + (long long)d1.n[0] * d1.n[1] * d1.n[2] * ncomp;
-    const T *ins[3] = {src, t1, t2};
-    T *outs[3] = {t1, t2, dst};
-    const Dims3 di[3] = {dc, d1, d2}, dd[3] = {d1, d2, df};
-    const int axes[3] = {2, 1, 0};
-    for (int p = 0; p < 3; ++p) {
-      if (vel)
-        hipLaunchKernelGGL((k_prolong_pass<2, T>), blocks(dd[p]), dim3(256), 0, st, Lc, Lf, axes[p], di[p], dd[p],
-                           ncomp, p == 0 ? 1 : 0, p == 2 ? 1 : 0, p == 2 && add ? 1 : 0, ins[p], outs[p]);
-      else
-        hipLaunchKernelGGL((k_prolong_pass<1, T>), blocks(dd[p]), dim3(256), 0, st, Lc, Lf, axes[p], di[p], dd[p],
-                           ncomp, 0, 0, p == 2 && add ? 1 : 0, ins[p], outs[p]);
-    }
-  }
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  if (Lf.dim == 3 && vel)
+    go(I3(), I2());
+  else if (Lf.dim == 3)
+    go(I3(), I1());
+  else if (vel)
+    go(I2(), I2());
+  else
+    go(I2(), I1());
   MFS_HIP(hipGetLastError());
-}
-long long transfer_work_size(const LevelDesc &Lc, const LevelDesc &Lf) {
-  // two work arrays: velocity (c, f, f) and (c, c, f) per component (restriction) or
-  // (c, c, f) and (c, f, f) (prolongation); sized for the larger of the two orders
-  const long long a = (long long)Lc.nv[0] * Lf.nv[1] * Lf.nv[2], b = (long long)Lc.nv[0] * Lc.nv[1] * Lf.nv[2];
-  return 3 * (a + b);
 }
 
 template <typename T>
 void launch_prolongate(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src_c, T *dst_f, bool add,
-                       hipStream_t st, T *work) {
-  if (work && Lf.k == 2) {
-    run_sep_transfer<T>(true, kind, Lc, Lf, src_c, dst_f, add, work, st);
+                       hipStream_t st) {
+  if (Lf.k == 2) {
+    run_cell_transfer<T>(true, kind, Lc, Lf, src_c, dst_f, add, st);
     return;
   }
   const long long n = kind == 0 ? Lf.vnodes : Lf.pnodes;
@@ -1989,9 +1962,9 @@ void launch_prolongate(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const
 }
 template <typename T>
 void launch_restrict(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src_f, T *dst_c,
-                     hipStream_t st, T *work) {
-  if (work && Lf.k == 2) {
-    run_sep_transfer<T>(false, kind, Lc, Lf, src_f, dst_c, false, work, st);
+                     hipStream_t st) {
+  if (Lf.k == 2) {
+    run_cell_transfer<T>(false, kind, Lc, Lf, src_f, dst_c, false, st);
     return;
   }
   const long long n = kind == 0 ? Lc.vnodes : Lc.pnodes;
@@ -2004,13 +1977,13 @@ void launch_restrict(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T
   MFS_HIP(hipGetLastError());
 }
 template void launch_prolongate<double>(int, const LevelDesc &, const LevelDesc &, const double *, double *, bool,
-                                        hipStream_t, double *);
+                                        hipStream_t);
 template void launch_prolongate<float>(int, const LevelDesc &, const LevelDesc &, const float *, float *, bool,
-                                       hipStream_t, float *);
+                                       hipStream_t);
 template void launch_restrict<double>(int, const LevelDesc &, const LevelDesc &, const double *, double *,
-                                      hipStream_t, double *);
+                                      hipStream_t);
 template void launch_restrict<float>(int, const LevelDesc &, const LevelDesc &, const float *, float *,
-                                     hipStream_t, float *);
+                                     hipStream_t);
 
 // ------------------------------------------------------------------ viscosity tables
 __device__ __forceinline__ long long tile_index(const LevelDesc &L, int gcx, int gcy, int gcz, int TX, int TY,

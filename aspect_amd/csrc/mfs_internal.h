@@ -213,15 +213,11 @@ bool launch_march_cheb(const LevelDesc &L, const T *x_in, const T *b, const T *e
                        T *x_out, T f1, T f2, int first, hipStream_t st);
 
 // Transfers between level Lc (coarse) and Lf = refined Lc.  kind 0 velocity, 1 pressure.
-// work: nullptr, or transfer_work_size(Lc, Lf) elements for the separable
-// (one direction per pass) 3D degree-2 path
 template <typename T>
 void launch_prolongate(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src_c, T *dst_f, bool add,
-                       hipStream_t st, T *work = nullptr);
+                       hipStream_t st);
 template <typename T>
-void launch_restrict(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src_f, T *dst_c,
-                     hipStream_t st, T *work = nullptr);
-long long transfer_work_size(const LevelDesc &Lc, const LevelDesc &Lf);
+void launch_restrict(int kind, const LevelDesc &Lc, const LevelDesc &Lf, const T *src_f, T *dst_c, hipStream_t st);
 
 // Pressure mass apply (degree 2, 2D or 3D box, cellwise viscosity) from a
 // natural-order table of inverse cell viscosities (launch_inv_eta_nat); false
