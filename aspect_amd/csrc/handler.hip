@@ -613,7 +613,7 @@ struct GMG {
   // in x.
   void smooth_schur_fused(GMGLevel<T> &g, const ChebInfo &ch, T *x, const T *b, bool x_zero, int steps) {
     const bool inner = ch.degree >= 2 && std::fabs(ch.delta) >= 1e-40;
-    {  // a level that fits one workgroup: the whole sequence in one launch
+    {  // several steps per launch
       MassChebSeq seq{};
       const double inv_theta = 1.0 / ch.theta;
       bool fits = true;
@@ -637,7 +637,7 @@ struct GMG {
           rho_old = rho;
         }
       }
-      if (fits && launch_mass_smooth_small<T>(g.L, x, b, g.dinvS.p, g.ietan.p, seq, x_zero, st)) return;
+      if (fits && launch_mass_sweeps<T>(g.L, x, g.pr.p, b, g.dinvS.p, g.ietan.p, seq, x_zero, st)) return;
     }
     int swaps = 0;
     for (int s = 0; s < steps; ++s) swaps += (x_zero && s == 0 ? 0 : 1) + (inner ? ch.degree - 1 : 0);
@@ -1532,8 +1532,6 @@ void create(const mfs_box *b, int prec, mfs_handle **out) {
     throw std::runtime_error("mfs_create: no HIP device available");
   upload_basis_tables();
   (void)noalloc_scratch();
-  static std::once_flag smoother_once;
-  std::call_once(smoother_once, init_small_smoother);
   auto h = std::make_unique<mfs_handle>();
   h->box = *b;
   for (int d = b->dim; d < 3; ++d) {

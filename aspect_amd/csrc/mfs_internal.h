@@ -239,14 +239,18 @@ struct MassChebSeq {
   double f1[MAX], f2[MAX];
   int first[MAX];
 };
-// LDS budget of the single-workgroup smoother (2 pressure vectors + cells)
-constexpr size_t kSmallSmoothLds = 144 * 1024;
-// The whole Schur smoothing of a degree-2 level that fits one workgroup's LDS
-// in one launch (x from zero when x_zero); false if the level does not fit
+// node-wise mass kernels apply: degree 2 (Q1 pressure), box geometry, 32-bit offsets
+inline bool mass_nodes_ok(const LevelDesc &L) {
+  if (L.k != 2 || L.geo) return false;
+  if (L.pnodes >= (1LL << 31) || L.ntiles_total * 64 >= (1LL << 31) || L.cells >= (1LL << 31))
+    throw std::runtime_error("level too large for the node-wise mass apply (32-bit offsets)");
+  return true;
+}
+// The Schur smoothing of a degree-2 level with several steps per launch, in x (in and
+// out; other is a second buffer); false where no sweep of seq fits a launch
 template <typename T>
-bool launch_mass_smooth_small(const LevelDesc &L, T *x, const T *b, const T *dinv, const T *ieta,
-                              const MassChebSeq &seq, bool x_zero, hipStream_t st);
-void init_small_smoother();
+bool launch_mass_sweeps(const LevelDesc &L, T *x, T *other, const T *b, const T *dinv, const T *ieta,
+                        const MassChebSeq &seq, bool x_zero, hipStream_t st);
 // B^T for degree 2 as a node-wise stencil (dst_u = op(B^T src_p) by mode, rhs_u
 // for RESID), computed in T and stored as TO; false for degree 3
 template <typename T, typename TO>
