@@ -78,17 +78,47 @@ __global__ void k_resolve(const long long n, const double *__restrict__ src, con
   out[i] = a;
 }
 
-// sum of the cell contributions of one node (component offset coff)
+// sum of the cell contributions of one node (component offset coff), in the
+// order of its list.  Eight at a time with their loads in flight together: a node
+// has at most 8 cells away from irregular corners, and one load after the other is a
+// chain of 16 latencies.
 __device__ __forceinline__ double node_sum(const double *__restrict__ cb, const long long *__restrict__ iptr,
                                            const int *__restrict__ ioff, long long node, long long coff) {
+  const long long end = iptr[node + 1];
   double a = 0;
-  for (long long k = iptr[node]; k < iptr[node + 1]; ++k) a += cb[ioff[k] + coff];
+  for (long long k = iptr[node]; k < end; k += 8) {
+    const int left = (int)min(end - k, 8LL);
+    int o[8];
+    double v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = j < left ? ioff[k + j] : 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = j < left ? cb[o[j] + coff] : 0.0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j < left) a += v[j];
+  }
   return a;
+}
+// the component of a DoF (at most 3 of nn nodes)
+__device__ __forceinline__ int component_of(long long dof, long long nn) {
+  return (dof >= nn ? 1 : 0) + (dof >= 2 * nn ? 1 : 0);
+}
+// sums of the constrained DoFs that have masters, one thread each, for
+// k_assemble to add to the masters
+__global__ void k_line_sums(const int n, const long long nn, const long long cs, const double *__restrict__ cb,
+                            const long long *__restrict__ iptr, const int *__restrict__ ioff,
+                            const long long *__restrict__ dof, double *__restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const long long i = dof[t];
+  const int comp = component_of(i, nn);
+  out[t] = node_sum(cb, iptr, ioff, i - comp * nn, comp * cs);
 }
 
 // dst[i] for the DoFs of one block (nn nodes per component, component stride
 // cs in the contribution buffer): free DoFs their own sum plus the weighted
-// sums of the constrained DoFs they are a master of; constrained DoFs
+// sums (k_line_sums) of the constrained DoFs they are a master of; constrained DoFs
 // src[i] (ident) or 0
 // Fused modes of the assemble pass (the smoother's steps on a level):
 // AS_RESID dst = b - K src; AS_CHEB one Jacobi-Chebyshev step on x = src (in
@@ -101,37 +131,64 @@ struct ChebStep {
   double f1, f2;  // first step: f2 = 1 / theta
   int first;
 };
+// Bound by chains of dependent gathers.  A master that summed the lists of its
+// constrained DoFs itself, one after the other, held its level up: on 1843 cells with
+// hanging nodes 31 us (velocity) and 12.5 us (pressure) against 8.7 + 4.6 us and 5.7 +
+// 3.8 us with the sums in a launch of their own, on 14.7k cells 52 us against 16 + 4.5 us. One
+// thread for the components of a node, sharing its list, was slower still (80 us, as the
+// lists of three DoFs followed each other).
 template <int MODE>
 __global__ void k_assemble(const long long n, const long long nn, const long long cs, const double *__restrict__ cb,
                            const long long *__restrict__ iptr, const int *__restrict__ ioff,
                            const int *__restrict__ row, const long long *__restrict__ tptr,
-                           const long long *__restrict__ tdof, const double *__restrict__ tw,
-                           const double *__restrict__ src, double *__restrict__ dst, const int ident,
-                           const ChebStep ch) {
+                           const int *__restrict__ tline, const double *__restrict__ tw,
+                           const double *__restrict__ sums, const double *__restrict__ src, double *__restrict__ dst,
+                           const int ident, const ChebStep ch) {
   // XCD-aware order: neighbouring nodes gather from the same cells' contribution
   // lines, so contiguous node ranges go to one XCD (one L2)
   const long long i = xcd_order(blockIdx.x, gridDim.x) * (long long)blockDim.x + threadIdx.x;
   if (i >= n) return;
+  // everything that does not wait for the node's list first
+  const int line = row[i];
+  const long long t0 = tptr[i], t1 = tptr[i + 1];
+  double bi = 0, di = 0, dold = 0, xi = 0;
+  if constexpr (MODE != AS_SET) bi = ch.b[i];
+  if constexpr (MODE == AS_CHEB) {
+    di = ch.dinv[i];
+    xi = src[i];
+    if (!ch.first) dold = ch.d[i];
+  }
   double a;
-  if (row[i] >= 0) {
+  if (line >= 0) {
     a = ident ? src[i] : 0.0;
   } else {
-    const long long comp = i / nn, node = i - comp * nn;
-    a = node_sum(cb, iptr, ioff, node, comp * cs);
-    for (long long k = tptr[i]; k < tptr[i + 1]; ++k) {
-      const long long c = tdof[k], cc = c / nn;
-      a += tw[k] * node_sum(cb, iptr, ioff, c - cc * nn, cc * cs);
+    const int comp = component_of(i, nn);
+    a = node_sum(cb, iptr, ioff, i - comp * nn, comp * cs);
+    for (long long k = t0; k < t1; k += 4) {
+      const int left = (int)min(t1 - k, 4LL);
+      int l[4];
+      double w[4], v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        l[j] = j < left ? tline[k + j] : 0;
+        w[j] = j < left ? tw[k + j] : 0.0;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = j < left ? sums[l[j]] : 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < left) a += w[j] * v[j];
     }
   }
   if constexpr (MODE == AS_SET) {
     dst[i] = a;
   } else if constexpr (MODE == AS_RESID) {
-    dst[i] = 1.0 * ch.b[i] + -1.0 * a;
+    dst[i] = 1.0 * bi + -1.0 * a;
   } else {
-    const double r = 1.0 * ch.b[i] + -1.0 * a;
-    const double dd = ch.first ? ch.dinv[i] * r * ch.f2 : ch.f1 * ch.d[i] + ch.f2 * ch.dinv[i] * r;
+    const double r = 1.0 * bi + -1.0 * a;
+    const double dd = ch.first ? di * r * ch.f2 : ch.f1 * dold + ch.f2 * di * r;
     ch.d[i] = dd;
-    dst[i] = src[i] + dd;
+    dst[i] = xi + dd;
   }
 }
 
@@ -186,27 +243,37 @@ __global__ void k_tria_mass_apply(const long long ncells, const int *__restrict_
   const long long c = xcd_order(blockIdx.x, gridDim.x) * (long long)blockDim.x + threadIdx.x;
   if (c >= ncells) return;
   const long long b = c / 64, cc = c - b * 64;
-  double p[NP], y[NP];
+  // the loads of all nodes and of the matrix in flight together, then the constrained nodes
+  // (a node after the other was a chain of 8 times 3 latencies)
+  double p[NP], y[NP], m[NT];
+  int node[NP], line[NP];
+#pragma unroll
+  for (int a = 0; a < NP; ++a) node[a] = cell_p[(b * NP + a) * 64 + cc];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) m[t] = mat[(b * NT + t) * 64 + cc];
+  bool lines = false;
 #pragma unroll
   for (int a = 0; a < NP; ++a) {
-    const int node = cell_p[(b * NP + a) * 64 + cc];
-    const int r = row[node];
-    double v;
-    if (r < 0) {
-      v = x[node];
-    } else {
-      v = 0;
-      for (long long k = off[r]; k < off[r + 1]; ++k) v += w[k] * x[mas[k]];
-    }
-    p[a] = v;
+    line[a] = row[node[a]];
+    p[a] = x[node[a]];
     y[a] = 0;
+  }
+#pragma unroll
+  for (int a = 0; a < NP; ++a) lines = lines || line[a] >= 0;
+  if (lines) {
+#pragma unroll
+    for (int a = 0; a < NP; ++a)
+      if (line[a] >= 0) {
+        p[a] = 0;
+        for (long long k = off[line[a]]; k < off[line[a] + 1]; ++k) p[a] += w[k] * x[mas[k]];
+      }
   }
   int t = 0;
 #pragma unroll
   for (int i = 0; i < NP; ++i)
 #pragma unroll
     for (int j = i; j < NP; ++j) {
-      const double v = mat[(b * NT + t++) * 64 + cc];
+      const double v = m[t++];
       y[i] += v * p[j];
       if (j != i) y[j] += v * p[i];
     }
@@ -218,8 +285,13 @@ __global__ void k_tria_mass_apply(const long long ncells, const int *__restrict_
 struct DevCon {
   long long n = 0;
   Buf<int> row;
-  Buf<long long> off, mas, tptr, tdof;
+  Buf<long long> off, mas, tptr;
   Buf<double> w, tw;
+  // constrained DoFs with masters, per transposed entry their index in that list, and their sums in an apply
+  int n_hang = 0;
+  Buf<long long> hang;
+  Buf<int> tline;
+  Buf<double> sums;
   std::vector<char> fixed;  // host copy: 1 on constrained DoFs
 
   // host-side check of the lines (no device call): DoFs and masters in range,
@@ -236,17 +308,22 @@ struct DevCon {
     mas.upload(h_mas, st);
     w.upload(h_w, st);
     tptr.upload(h_tptr, st);
-    tdof.upload(h_tdof, st);
+    tline.upload(h_tline, st);
+    hang.upload(h_hang, st);
+    n_hang = (int)h_hang.size();
+    sums.alloc(h_hang.size());
     tw.upload(h_tw, st);
     MFS_HIP(hipStreamSynchronize(st));
     h_w.clear();
     h_tptr.clear();
-    h_tdof.clear();
+    h_tline.clear();
+    h_hang.clear();
     h_tw.clear();
   }
 
   std::vector<int> h_row;
-  std::vector<long long> h_off, h_mas, h_tptr, h_tdof;
+  std::vector<long long> h_off, h_mas, h_tptr, h_hang;
+  std::vector<int> h_tline;
   std::vector<double> h_w, h_tw;
 
   void build(long long ndof, const mfs_constraints *c, const char *what) {
@@ -286,21 +363,26 @@ struct DevCon {
       }
       o.push_back((long long)m.size());
     }
-    // transpose: for every master, the (constrained DoF, weight) pairs, in line order
-    std::vector<long long> &tp = h_tptr, &td = h_tdof;
+    // transpose: for every master, the (constrained DoF, weight) pairs, in line
+    // order, a DoF as its index in the list of those with masters
+    std::vector<long long> &tp = h_tptr;
+    std::vector<int> &tl = h_tline;
     std::vector<double> &tv = h_tw;
+    h_hang.clear();
     tp.assign(ndof + 1, 0);
-    td.assign(m.size(), 0);
+    tl.assign(m.size(), 0);
     tv.assign(m.size(), 0.0);
     for (long long k = 0; k < (long long)m.size(); ++k) ++tp[m[k] + 1];
     for (long long i = 0; i < ndof; ++i) tp[i + 1] += tp[i];
     std::vector<long long> fill(tp.begin(), tp.end() - 1);
-    for (long long l = 0; l < nl; ++l)
+    for (long long l = 0; l < nl; ++l) {
       for (long long k = o[l]; k < o[l + 1]; ++k) {
         const long long pos = fill[m[k]]++;
-        td[pos] = c->dofs[l];
+        tl[pos] = (int)h_hang.size();
         tv[pos] = ww[k];
       }
+      if (o[l + 1] > o[l]) h_hang.push_back(c->dofs[l]);
+    }
   }
 };
 
@@ -462,15 +544,19 @@ struct mfs_tria {
                 DevCon &c, const double *src, double *dst, int ident, hipStream_t s, int mode = AS_SET,
                 const ChebStep &ch = ChebStep{}) {
     const unsigned nb = (unsigned)((c.n + 255) / 256);
+    if (c.n_hang > 0)
+      hipLaunchKernelGGL(k_line_sums, dim3((unsigned)((c.n_hang + 63) / 64)), dim3(64), 0, s, c.n_hang, nn, cs, cb, ip.p,
+                         io.p, c.hang.p, c.sums.p);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, s, c.n, nn, cs, cb, ip.p, io.p, c.row.p, c.tptr.p, c.tline.p,
+                         c.tw.p, c.sums.p, src, dst, ident, ch);
+    };
     if (mode == AS_SET)
-      hipLaunchKernelGGL(k_assemble<AS_SET>, dim3(nb), dim3(256), 0, s, c.n, nn, cs, cb, ip.p, io.p, c.row.p,
-                         c.tptr.p, c.tdof.p, c.tw.p, src, dst, ident, ch);
+      go(k_assemble<AS_SET>);
     else if (mode == AS_RESID)
-      hipLaunchKernelGGL(k_assemble<AS_RESID>, dim3(nb), dim3(256), 0, s, c.n, nn, cs, cb, ip.p, io.p, c.row.p,
-                         c.tptr.p, c.tdof.p, c.tw.p, src, dst, ident, ch);
+      go(k_assemble<AS_RESID>);
     else
-      hipLaunchKernelGGL(k_assemble<AS_CHEB>, dim3(nb), dim3(256), 0, s, c.n, nn, cs, cb, ip.p, io.p, c.row.p,
-                         c.tptr.p, c.tdof.p, c.tw.p, src, dst, ident, ch);
+      go(k_assemble<AS_CHEB>);
     MFS_HIP(hipGetLastError());
   }
 
