@@ -8,13 +8,19 @@
 //
 // On a uniform level with one viscosity per cell the cell operator is the
 // viscosity times one constant matrix (81 x 81 in 3D).  The cell is symmetric
-// under reflection in each direction, so in the basis of sums and differences
-// of opposite nodes (per direction e0 = a + c, e1 = b, o = a - c) that matrix
-// splits into blocks of equal symmetry: 855 non-zeros instead of 6561 in 3D (82
+// under reflection in each direction, so in the basis of differences of
+// opposite nodes (per direction a - 2 b + c, b, a - c) that matrix
+// splits into blocks of equal symmetry: 795 entries instead of 6561 in 3D (64
 // instead of 324 in 2D), B^T and B into one entry per velocity mode.  That is
 // 3.5 times less arithmetic than the sum factorization over quadrature points
 // and needs no quadrature data.  The integrals are exact, as the Gauss rule's
-// are (degree 4 in each direction).
+// are (degree 4 in each direction).  A constant is the mode b in all
+// directions, whose entries vanish: applied to a constant the operator gives
+// zero to the last bit.  With a + c for a - 2 b + c it did so only up to the
+// rounding of the entries, the same in every cell: 15 GMRES steps on 12 2D
+// problems of 16^2 to 128^2 cells then ended 1.9e-13 to 2.9e-13 from the
+// result of 64 bits, now 1.5e-14 to 3.6e-14 (from quadrature 5e-14 to 1e-13),
+// at the same speed.
 //
 // A workgroup owns the nodes of a box of cells and computes every cell that
 // touches them, so each node is finished by one thread: no work array, no
@@ -30,7 +36,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -45,25 +50,29 @@ namespace {
 
 constexpr int MARCH_CHEB = 3;  // besides MODE_SET / RESID / ADD
 
-// 1D tables of the quadratic basis on [0, 1] (nodes 0, 1/2, 1) and the linear
-// one (nodes 0, 1): mass, stiffness, derivative times value, and the two
-// products with the linear basis
-constexpr long double kM[3][3] = {{4.0L / 30, 2.0L / 30, -1.0L / 30}, {2.0L / 30, 16.0L / 30, 2.0L / 30}, {-1.0L / 30, 2.0L / 30, 4.0L / 30}};
-constexpr long double kL[3][3] = {{7.0L / 3, -8.0L / 3, 1.0L / 3}, {-8.0L / 3, 16.0L / 3, -8.0L / 3}, {1.0L / 3, -8.0L / 3, 7.0L / 3}};
-constexpr long double kC[3][3] = {{-1.0L / 2, -2.0L / 3, 1.0L / 6}, {2.0L / 3, 0, -2.0L / 3}, {-1.0L / 6, 2.0L / 3, 1.0L / 2}};
-constexpr long double kPM[3][2] = {{1.0L / 6, 0}, {1.0L / 3, 1.0L / 3}, {0, 1.0L / 6}};
-constexpr long double kPD[3][2] = {{-5.0L / 6, -1.0L / 6}, {2.0L / 3, -2.0L / 3}, {1.0L / 6, 5.0L / 6}};
-// nodal values from the sums and differences: a = (e0 + o) / 2, b = e1, c = (e0 - o) / 2
-constexpr long double kInv[3][3] = {{.5, 0, .5}, {0, 1, 0}, {.5, 0, -.5}};
-constexpr long double kInvP[2][2] = {{.5, .5}, {.5, -.5}};
+// 1D integrals over [0, 1] of the modes of the quadratic basis (nodes 0, 1/2, 1
+// with values a, b, c): modes a - 2 b + c, b and a - c, whose functions are
+// (1 - 2x)^2 / 2, 1 and (1 - 2x) / 2; and of the linear basis' modes a + c and
+// a - c with functions 1 / 2 and (1 - 2x) / 2.  Mass, stiffness, derivative
+// times value, and the two products with the linear basis.  The derivative of
+// mode 1 is zero: a constant has exactly no strain, however the other entries
+// are rounded.  (With modes a + c, b, a - c the entries cancel for a constant
+// only up to their rounding, the same in every cell of a level, which acts like
+// a small mass term and which a solve amplifies with the condition of the level.)
+constexpr long double kM[3][3] = {{1.0L / 20, 1.0L / 6, 0}, {1.0L / 6, 1, 0}, {0, 0, 1.0L / 12}};
+constexpr long double kK[3][3] = {{4.0L / 3, 0, 0}, {0, 0, 0}, {0, 0, 1}};
+constexpr long double kD[3][3] = {{0, 0, -1.0L / 3}, {0, 0, 0}, {-1.0L / 6, -1, 0}};
+constexpr long double kPM[3][2] = {{1.0L / 12, 0}, {1.0L / 2, 0}, {0, 1.0L / 12}};
+constexpr long double kPD[3][2] = {{0, -1.0L / 3}, {0, 0}, {-1.0L / 2, 0}};
 
 // modes 0, 1 are even, mode 2 is odd
 constexpr __host__ __device__ int par(int m) { return m == 2; }
 
 // 2D: does the block (output component c, input component d) couple output
 // mode m with input mode q?  The parities agree in both directions, or differ
-// in both for an off-diagonal block
+// in both for an off-diagonal block; the constant (mode 1 in both directions) couples with none
 constexpr __host__ __device__ bool couples2(int c, int d, int m, int q) {
+  if (m == 4 || q == 4) return false;
   const bool x = par(m % 3) == par(q % 3), y = par(m / 3) == par(q / 3);
   return c == d ? x && y : !x && !y;
 }
@@ -73,7 +82,7 @@ constexpr __host__ __device__ int pressure_mode2(int c, int m) { return (par(m %
 // 2D coefficients per output component c: the blocks of the input components c
 // and c + 1 (mod 2), input mode by input mode, then the B^T entry of every mode.
 struct March2 {
-  static constexpr int NM = 9, BLOCK = 25 + 16, STRIDE = BLOCK + NM;
+  static constexpr int NM = 9, STRIDE = 18 + 14 + NM;
 };
 
 // 3D coefficients per output component c, in register rows of 16 (k_march3).
@@ -81,11 +90,13 @@ struct March2 {
 // 9 m_{c+2}, directions mod 3), so that one code serves every component.  The
 // blocks of the input components c, c + 1, c + 2, each by symmetry class of its
 // input modes, every input of a class with every output of the
-// class it couples with.  The products of class sizes are powers of two; by
-// size the diagonal block fills 4 + 3 rows and one of 4 + 4 + 4 + 1, another
-// block 4 rows and one of 4 x 4; then B^T by class: 8 + 4 + 4, 4 + 2 + 2 + 2 + 1.
+// class it couples with.  The products of class sizes are powers of two.  Class 0
+// of the diagonal block, even in all directions, leaves out what vanishes
+// (class0_in): 2 rows and 12 places.  By size the diagonal block fills 2 rows,
+// one of 12 + 4, 3 rows and one of 4 + 4 + 1, another block 4 rows and one of
+// 4 x 4; then B^T by class: 8 + 4 + 4, 4 + 2 + 2 + 2 + 1.
 struct March3 {
-  static constexpr int ROWS = 18, STRIDE = (ROWS + 2) * 16;
+  static constexpr int ROWS = 17, STRIDE = (ROWS + 2) * 16;
 };
 // k-th symmetry class (bit e: odd in direction e) in table order; the diagonal
 // block's order also is the B^T rows' order
@@ -114,6 +125,17 @@ constexpr __host__ __device__ int class_mode(int cls, int j) {
   }
   return m;
 }
+// Class 0 of the diagonal block: an entry needs a direction in which both modes
+// have a derivative (index bit 0 of that direction).  The i-th input: four that
+// couple with all outputs, then three with one such direction, each with the four
+// outputs that have it too; the constant with none.  Its j-th output
+constexpr __host__ __device__ int class0_in(int i) {
+  constexpr int in[7] = {0, 1, 2, 4, 3, 5, 6};
+  return in[i];
+}
+constexpr __host__ __device__ int class0_out(int i, int j) {
+  return i < 4 ? j : (i == 4 ? j : (i == 5 ? (j & 1) | (j & 2) << 1 : j << 1));
+}
 // m: mode numbered from direction c on; the same mode numbered from direction 0 on
 constexpr __host__ __device__ int mode_from0(int c, int m) {
   constexpr int t[3] = {1, 3, 9};
@@ -123,8 +145,8 @@ constexpr __host__ __device__ int mode_from0(int c, int m) {
 constexpr __host__ __device__ int mode_from(int c, int m) { return mode_from0((3 - c) % 3, m); }
 // first lane, over the rows, of class k of block r (input component c + r)
 constexpr __host__ __device__ int class_lane(int r, int k) {
-  constexpr int diag[8] = {0, 64, 80, 96, 112, 116, 120, 124};
-  return r == 0 ? diag[k] : 128 + 80 * (r - 1) + (k < 4 ? 16 * k : 64 + 4 * (k - 4));
+  constexpr int diag[8] = {0, 48, 64, 80, 44, 96, 100, 104};
+  return r == 0 ? diag[k] : 112 + 80 * (r - 1) + (k < 4 ? 16 * k : 64 + 4 * (k - 4));
 }
 // first lane of class k in the B^T rows
 constexpr __host__ __device__ int bt_lane(int k) {
@@ -132,34 +154,15 @@ constexpr __host__ __device__ int bt_lane(int k) {
   return lane[k];
 }
 
-// exact integrals of a cell's modes
+// integrals of a cell's modes
 struct CellIntegrals {
   const LevelDesc &L;
-  long double M[3][3] = {}, K[3][3] = {}, D[3][3] = {}, PM[3][2] = {}, PD[3][2] = {};
-  explicit CellIntegrals(const LevelDesc &l) : L(l) {
-    for (int a = 0; a < 3; ++a)
-      for (int i = 0; i < 3; ++i) {
-        for (int b = 0; b < 3; ++b)
-          for (int j = 0; j < 3; ++j) {
-            const long double w = kInv[i][a] * kInv[j][b];
-            M[a][b] += w * kM[i][j];
-            K[a][b] += w * kL[i][j];
-            D[a][b] += w * kC[i][j];
-          }
-        for (int b = 0; b < 2; ++b)
-          for (int j = 0; j < 2; ++j) {
-            const long double w = kInv[i][a] * kInvP[j][b];
-            PM[a][b] += w * kPM[i][j];
-            PD[a][b] += w * kPD[i][j];
-          }
-      }
-  }
   // int d_a phi_m d_b phi_q over the cell
   long double grad(int a, int b, int m, int q) const {
     long double v = (long double)L.vol * L.ih[a] * L.ih[b];
     for (int e = 0, s = 1; e < L.dim; ++e, s *= 3) {
       const int i = m / s % 3, j = q / s % 3;
-      v *= e == a ? (e == b ? K[i][j] : D[i][j]) : (e == b ? D[j][i] : M[i][j]);
+      v *= e == a ? (e == b ? kK[i][j] : kD[i][j]) : (e == b ? kD[j][i] : kM[i][j]);
     }
     return v;
   }
@@ -176,68 +179,22 @@ struct CellIntegrals {
     long double v = -(long double)L.vol * L.ih[c];
     for (int e = 0, t = 1; e < L.dim; ++e, t *= 3) {
       const int i = m / t % 3, j = s >> e & 1;
-      v *= e == c ? PD[i][j] : PM[i][j];
+      v *= e == c ? kPD[i][j] : kPM[i][j];
     }
     return v;
   }
 };
 
-// Entries of one output mode for a set of input modes, rounded to T.  A constant
-// velocity has no strain, so the entries times the modes of the constant (2 for
-// a mode 0, 1 for a mode 1 in each direction) sum to zero; independent rounding
-// would leave a remainder, the same in every cell, which acts like a small mass
-// term and is amplified by the condition of the level in a solve (2D solves:
-// 3e-10 instead of 1e-12 from the exact result).  The remainder goes into the
-// entries, from the largest on to ever finer last places.
-template <typename T>
-void round_entries(const CellIntegrals &I, int c, int m, int d, const std::vector<int> &q, T *out, int stride) {
-  std::vector<size_t> order;
-  std::vector<long double> w;  // the constant's modes
-  long double sum = 0;
-  bool even = true;
-  for (size_t i = 0; i < q.size(); ++i) {
-    out[i * stride] = (T)I.block(c, m, d, q[i]);
-    order.push_back(i);
-    w.push_back(1);
-    for (int e = 0, t = 1; e < I.L.dim; ++e, t *= 3) {
-      if (q[i] / t % 3 == 0) w.back() *= 2;
-      even = even && q[i] / t % 3 != 2;
-    }
-    sum += w.back() * (long double)out[i * stride];
-  }
-  if (!even) return;  // the constant has no odd modes
-  std::stable_sort(order.begin(), order.end(),
-                   [&](size_t a, size_t b) { return std::fabs(out[a * stride]) > std::fabs(out[b * stride]); });
-  for (const size_t i : order) {
-    T &v = out[i * stride];
-    const T old = v;
-    v = (T)((long double)v - sum / w[i]);
-    sum += w[i] * ((long double)v - (long double)old);
-  }
-}
-
 template <typename T>
 void cell_tables2(const CellIntegrals &I, std::vector<T> &out) {
   out.assign(2 * March2::STRIDE, (T)0);
   for (int c = 0; c < 2; ++c) {
-    T *const row = out.data() + c * March2::STRIDE;
-    int at = 0;
-    for (int r = 0; r < 2; ++r) {
-      // entry positions, input mode by input mode
-      const int d = (c + r) % 2;
-      int pos[9][9];
+    T *at = out.data() + c * March2::STRIDE;
+    for (int r = 0; r < 2; ++r)
       for (int q = 0; q < March2::NM; ++q)
-        for (int m = 0; m < March2::NM; ++m) pos[m][q] = couples2(c, d, m, q) ? at++ : -1;
-      for (int m = 0; m < March2::NM; ++m) {
-        std::vector<int> q;
-        for (int j = 0; j < March2::NM; ++j)
-          if (pos[m][j] >= 0) q.push_back(j);
-        std::vector<T> v(q.size());
-        round_entries<T>(I, c, m, d, q, v.data(), 1);
-        for (size_t i = 0; i < q.size(); ++i) row[pos[m][q[i]]] = v[i];
-      }
-    }
-    for (int m = 0; m < March2::NM; ++m) row[March2::BLOCK + m] = (T)I.bt(c, m, pressure_mode2(c, m));
+        for (int m = 0; m < March2::NM; ++m)
+          if (couples2(c, (c + r) % 2, m, q)) *at++ = (T)I.block(c, m, (c + r) % 2, q);
+    for (int m = 0; m < March2::NM; ++m) *at++ = (T)I.bt(c, m, pressure_mode2(c, m));
   }
 }
 template <typename T>
@@ -245,16 +202,16 @@ void cell_tables3(const CellIntegrals &I, std::vector<T> &out) {
   out.assign(3 * March3::STRIDE, (T)0);
   for (int c = 0; c < 3; ++c) {
     T *const row = out.data() + c * March3::STRIDE;
-    for (int r = 0; r < 3; ++r) {
-      const int d = (c + r) % 3;
+    for (int r = 0; r < 3; ++r)
       for (int k = 0; k < 8; ++k) {
-        const int in = class_at(0, r, k), to = class_out(0, r, in), no = class_size(to);
-        std::vector<int> q;
-        for (int i = 0; i < class_size(in); ++i) q.push_back(mode_from0(c, class_mode(in, i)));
-        for (int o = 0; o < no; ++o)
-          round_entries<T>(I, c, mode_from0(c, class_mode(to, o)), d, q, row + class_lane(r, k) + o, no);
+        const int in = class_at(0, r, k), to = class_out(0, r, in);
+        const bool c0 = r == 0 && k == 0;
+        T *at = row + class_lane(r, k);
+        for (int i = 0; i < (c0 ? 7 : class_size(in)); ++i)
+          for (int o = 0; o < (c0 && i > 3 ? 4 : class_size(to)); ++o)
+            *at++ = (T)I.block(c, mode_from0(c, class_mode(to, c0 ? class0_out(i, o) : o)), (c + r) % 3,
+                               mode_from0(c, class_mode(in, c0 ? class0_in(i) : i)));
       }
-    }
     for (int k = 0; k < 8; ++k) {
       const int cls = class_at(0, 0, k), s = cls ^ 1;  // pressure mode, numbered from direction c on
       for (int j = 0; j < class_size(cls); ++j)
@@ -269,7 +226,7 @@ void cell_tables3(const CellIntegrals &I, std::vector<T> &out) {
 bool march_level(const LevelDesc &L) { return L.k == 2; }
 template <typename T>
 std::vector<T> march_tables(const LevelDesc &L) {
-  const CellIntegrals I(L);
+  const CellIntegrals I{L};
   std::vector<T> t;
   if (L.dim == 3)
     cell_tables3<T>(I, t);
@@ -344,21 +301,21 @@ __device__ __forceinline__ T keep_if(unsigned m, int k, T v) {
     return __longlong_as_double(__double_as_longlong(v) & (long long)all);
 }
 
-// sums and differences along x and y of a 3 x 3 node plane [3 j + i]
+// modes of three node values a, b, c: a - 2 b + c, b, a - c.  The differences
+// of neighbours come first: they are exact where the field is smooth
+template <typename T>
+__device__ __forceinline__ void line_modes(T &a, const T b, T &c) {
+  const T l = a - b, r = c - b;
+  c = a - c;
+  a = l + r;
+}
+// modes along x and y of a 3 x 3 node plane [3 j + i]
 template <typename T>
 __device__ __forceinline__ void plane_modes(T (&p)[9]) {
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    const T a = p[3 * j], c = p[3 * j + 2];
-    p[3 * j] = a + c;
-    p[3 * j + 2] = a - c;
-  }
+  for (int j = 0; j < 3; ++j) line_modes<T>(p[3 * j], p[3 * j + 1], p[3 * j + 2]);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const T a = p[i], c = p[6 + i];
-    p[i] = a + c;
-    p[6 + i] = a - c;
-  }
+  for (int i = 0; i < 3; ++i) line_modes<T>(p[i], p[3 + i], p[6 + i]);
 }
 // tested modes of a cell's node plane to the sums at the cell's own four nodes
 // (i, j in {0, 1}), with the left and lower neighbours' shares
@@ -368,12 +325,12 @@ __device__ __forceinline__ void plane_nodes(const T (&y)[9], int below, T (&o)[2
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
     n[0][m] = y[3 * m] + y[3 * m + 2] + lane_left<T>(y[3 * m] - y[3 * m + 2]);
-    n[1][m] = y[3 * m + 1];
+    n[1][m] = y[3 * m + 1] - 2 * y[3 * m];
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     o[0][i] = n[i][0] + n[i][2] + lane_at<T>(below, n[i][0] - n[i][2]);
-    o[1][i] = n[i][1];
+    o[1][i] = n[i][1] - 2 * n[i][0];
   }
 }
 
@@ -462,26 +419,50 @@ __device__ __forceinline__ void fmac_group(const T k, const T *x, T *a) {
 }
 
 // Everything below is numbered from the output component's direction on.
+// acc += class 0 of the diagonal block
+template <int I, typename T>
+__device__ __forceinline__ void apply_class0_input(const T k, const T x, T (&acc)[27]) {
+  T a[4];
+#pragma unroll
+  for (int o = 0; o < 4; ++o) a[o] = acc[class_mode(0, class0_out(I, o))];
+  fmac_group<1, 4, 4 * (I - 4), T>(k, &x, a);
+#pragma unroll
+  for (int o = 0; o < 4; ++o) acc[class_mode(0, class0_out(I, o))] = a[o];
+}
+template <typename T>
+__device__ __forceinline__ void apply_class0(const T *k, const T *comp, T (&acc)[27]) {
+  T u[7], a[8];
+#pragma unroll
+  for (int i = 0; i < 7; ++i) u[i] = comp[class_mode(0, class0_in(i)) * 64];
+#pragma unroll
+  for (int o = 0; o < 8; ++o) a[o] = acc[class_mode(0, o)];
+  fmac_group<2, 8, 0, T>(k[0], u, a);
+  fmac_group<2, 8, 0, T>(k[1], u + 2, a);
+#pragma unroll
+  for (int o = 0; o < 8; ++o) acc[class_mode(0, o)] = a[o];
+  apply_class0_input<4, T>(k[2], u[4], acc);
+  apply_class0_input<5, T>(k[2], u[5], acc);
+  apply_class0_input<6, T>(k[2], u[6], acc);
+}
 // acc += block R of the modes of component R, which are stored numbered from
 // direction R on (comp: the column's entries), from class K on; k: coefficients
 // by register row
 template <int R, int K, typename T>
 __device__ __forceinline__ void apply_block(const T *k, const T *comp, T (&acc)[27]) {
-  constexpr int in = class_at(0, R, K), to = class_out(0, R, in);
-  constexpr int I = class_size(in), O = class_size(to), lane = class_lane(R, K);
-  T u[I], a[O];
-#pragma unroll
-  for (int i = 0; i < I; ++i) u[i] = comp[mode_from(R, class_mode(in, i)) * 64];
-#pragma unroll
-  for (int o = 0; o < O; ++o) a[o] = acc[class_mode(to, o)];
-  if constexpr (I * O == 64) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) fmac_group<2, 8, 0, T>(k[lane / 16 + r], u + 2 * r, a);
+  if constexpr (R == 0 && K == 0) {
+    apply_class0<T>(k, comp, acc);
   } else {
-    fmac_group<I, O, lane % 16, T>(k[lane / 16], u, a);
-  }
+    constexpr int in = class_at(0, R, K), to = class_out(0, R, in);
+    constexpr int I = class_size(in), O = class_size(to), lane = class_lane(R, K);
+    T u[I], a[O];
 #pragma unroll
-  for (int o = 0; o < O; ++o) acc[class_mode(to, o)] = a[o];
+    for (int i = 0; i < I; ++i) u[i] = comp[mode_from(R, class_mode(in, i)) * 64];
+#pragma unroll
+    for (int o = 0; o < O; ++o) a[o] = acc[class_mode(to, o)];
+    fmac_group<I, O, lane % 16, T>(k[lane / 16], u, a);
+#pragma unroll
+    for (int o = 0; o < O; ++o) acc[class_mode(to, o)] = a[o];
+  }
   if constexpr (K < 7) apply_block<R, K + 1, T>(k, comp, acc);
 }
 // acc[m] += b[m] * (pressure mode of its class), from class K on
@@ -511,9 +492,11 @@ template <int C, typename T>
 __device__ __forceinline__ void store_modes(const T (&lo)[9], const T (&mid)[9], const T (&hi)[9], T *to) {
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    to[mode_from(C, k) * 64] = lo[k] + hi[k];
+    T a = lo[k], c = hi[k];
+    line_modes<T>(a, mid[k], c);
+    to[mode_from(C, k) * 64] = a;
     to[mode_from(C, 9 + k) * 64] = mid[k];
-    to[mode_from(C, 18 + k) * 64] = lo[k] - hi[k];
+    to[mode_from(C, 18 + k) * 64] = c;
   }
 }
 // tested modes of component C to its node planes: lower (with the share carried
@@ -524,7 +507,7 @@ __device__ __forceinline__ void split_planes(const T (&acc)[27], T (&y)[2][9], T
   for (int q = 0; q < 9; ++q) {
     const T e = acc[mode_from(C, q)], o = acc[mode_from(C, 18 + q)];
     y[0][q] = e + o + carry[q];
-    y[1][q] = acc[mode_from(C, 9 + q)];
+    y[1][q] = acc[mode_from(C, 9 + q)] - 2 * e;
     carry[q] = e - o;
   }
 }

@@ -68,6 +68,23 @@ def test_stokes_2d_matches_oracle(n):
     assert np.linalg.norm(h.stokes_vmult(x) - ref) < TOL["fp64"] * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("compressible", [False, True])
+@pytest.mark.parametrize("n", [(9, 8, 10), (40, 33, 24), (1, 1, 1), (17, 9), (50, 3)])
+def test_constant_velocity_has_no_strain(n, compressible, prec):
+    # exactly zero, without a remainder of rounded entries: it would be the same in every
+    # cell of a level, like a small mass term
+    h, s, rng = _box(n, (0,) * (2 * len(n)), compressible, prec)
+    print("constant", n, prec, compressible, flush=True)
+    value = torch.tensor(rng.normal(size=(len(n), 1)), dtype=torch.float64 if prec == "fp64" else torch.float32, device="cuda:0")
+    x = value.expand(len(n), s["nu"] // len(n)).reshape(-1).contiguous()
+    y = torch.full_like(x, float("nan"))
+    torch.cuda.synchronize()
+    h.ablock_vmult_device(0, x.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    assert bool((y == 0).all())
+
+
 def test_source_outside_the_mesh_is_not_read_into_rows():
     # columns beyond the mesh read the nearest cells and discard the values:
     # an infinity at one node reaches only the rows of the cells that hold it
