@@ -143,16 +143,33 @@ LevelDesc make_level_desc(const mfs_box &b, int l) {
   return L;
 }
 
-// device copy of a level's cell matrices, referred to by its descriptor
-template <typename T>
-void attach_cell_matrices(LevelDesc &L, DBuf<T> &buf) {
-  if (!march_level(L)) return;
-  const std::vector<T> v = march_tables<T>(L);
-  buf.alloc((long long)v.size());
-  MFS_HIP(hipMemcpy(buf.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-  L.kmat = buf.p;
-  L.kmat_size = (int)sizeof(T);
-}
+// Cell matrices of a degree-2 box's levels (LevelDesc::kmat) on the device, in
+// each precision from the first viscosity of one value per cell on, kept with the
+// handle (made for every level and hierarchy, they were a fifth of the set-up of a small box)
+struct CellMatrices {
+  DBuf<double> d;
+  DBuf<float> f;
+  template <typename T>
+  void attach(LevelDesc &L, int level, const LevelDesc &L0, int n_levels, hipStream_t st) {
+    if (!march_level(L) || L.geo) return;
+    DBuf<T> *buf;
+    if constexpr (std::is_same<T, double>::value)
+      buf = &d;
+    else
+      buf = &f;
+    if (!buf->p) {
+      const std::vector<T> v = march_tables<T>(L0, n_levels);
+      DBuf<T> b;
+      b.alloc((long long)v.size());
+      MFS_HIP(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
+      MFS_HIP(hipStreamSynchronize(st));
+      std::swap(buf->p, b.p);
+      std::swap(buf->n, b.n);
+    }
+    L.kmat = buf->p + buf->n / n_levels * level;
+    L.kmat_size = (int)sizeof(T);
+  }
+};
 
 int n_qp(const mfs_box &b) {
   const int q = b.degree + 1;
@@ -174,7 +191,6 @@ struct GMGLevel {
   LevelDesc L;
   long long nu = 0, np = 0;
   DBuf<T> eta, dinvA, dinvS;
-  DBuf<T> kmat;   // cell matrices of a degree-2 level (LevelDesc::kmat)
   DBuf<T> ietan;  // 1 / cellwise viscosity in natural cell order (Schur level operator), set by build()
   DBuf<T> ux, ub, ur, ud, px, pb, pr, pd;
   ChebInfo chA, chS;
@@ -185,6 +201,7 @@ struct GMG {
   hipStream_t st;
   std::vector<std::unique_ptr<GMGLevel<T>>> lv;
   DBuf<double> *dot_work = nullptr, *dot_out = nullptr;
+  CellMatrices *cells = nullptr;  // the handle's; none in the mesh-deformation hierarchy
   int top = 0;
   // V-cycles replayed from a captured hipGraph (one per kind); the capture
   // holds kernel arguments (buffers, Chebyshev coefficients), so it is dropped
@@ -231,9 +248,10 @@ struct GMG {
   GMG &operator=(const GMG &) = delete;
   ~GMG() { drop_graphs(); }
 
-  void setup(const mfs_box &b, hipStream_t s, DBuf<double> *work, DBuf<double> *out) {
+  void setup(const mfs_box &b, hipStream_t s, DBuf<double> *work, DBuf<double> *out, CellMatrices *matrices = nullptr) {
     drop_graphs();
     st = s;
+    cells = matrices;
     dot_work = work;
     dot_out = out;
     lv.clear();
@@ -241,7 +259,6 @@ struct GMG {
     for (int l = 0; l < b.n_levels; ++l) {
       auto g = std::make_unique<GMGLevel<T>>();
       g->L = make_level_desc(b, l);
-      if (!laplace) attach_cell_matrices<T>(g->L, g->kmat);
       g->nu = (long long)b.dim * g->L.vnodes;
       g->np = g->L.pnodes;
       g->eta.alloc(g->L.ntiles_total * ct);
@@ -269,6 +286,8 @@ struct GMG {
     eta_pq = 0;
     eta_src = active;
     eta_src_pq = active_per_qp;
+    if (cells)
+      for (int l = 0; l <= top; ++l) cells->attach<T>(lv[l]->L, l, lv[0]->L, top + 1, st);
     for (auto &g : lv)
       if (g->eta.n != g->L.ntiles_total * cells_per_tile_of(g->L)) g->eta.alloc(g->L.ntiles_total * cells_per_tile_of(g->L));
     GMGLevel<T> &f = *lv[top];
@@ -498,7 +517,7 @@ struct GMG {
     shadow.reset();
     auto sh = std::make_unique<GMG<double>>();
     sh->graphs = false;
-    sh->setup(b, st, dot_work, dot_out);
+    sh->setup(b, st, dot_work, dot_out, cells);
     for (int l = 0; l <= top; ++l) sh->lv[l]->L.geo = lv[l]->L.geo;
     if (eta_pq)
       sh->set_eta_q1(*q1_src, q1_lo, q1_hi);
@@ -743,6 +762,7 @@ struct mfs_handle {
   int active_per_qp = 0;
   bool have_eta = false, have_prec = false;
   double eta_min = 0, eta_max = 0;
+  CellMatrices cells;
   GMG<float> g32;
   GMG<double> g64;
   DBuf<double> dot_work, dot_out, hbuf;
@@ -760,7 +780,6 @@ struct mfs_handle {
   std::vector<DBuf<double>> geo_lv;
   // work array of the split FP64 Stokes apply on the active level (3D degree 2)
   DBuf<double> swork_stokes;
-  DBuf<double> kmat_top;  // the active level's cell matrices
 
   ~mfs_handle() {
     for (double *p : vchunks) (void)hipFree(p);
@@ -1542,7 +1561,6 @@ void create(const mfs_box *b, int prec, mfs_handle **out) {
   MFS_HIP(hipStreamCreateWithFlags(&h->st, hipStreamNonBlocking));
   for (int l = 0; l < b->n_levels; ++l) h->L.push_back(make_level_desc(h->box, l));
   h->top = b->n_levels - 1;
-  attach_cell_matrices<double>(h->L[h->top], h->kmat_top);
   h->nu = (long long)b->dim * h->Ltop().vnodes;
   h->np = h->Ltop().pnodes;
   h->n = h->nu + h->np;
@@ -1556,9 +1574,9 @@ void create(const mfs_box *b, int prec, mfs_handle **out) {
     v_fill<double>(v->p, 0.0, v->n, h->st);
   }
   if (prec == MFS_GMG_FP32)
-    h->g32.setup(h->box, h->st, &h->dot_work, &h->dot_out);
+    h->g32.setup(h->box, h->st, &h->dot_work, &h->dot_out, &h->cells);
   else
-    h->g64.setup(h->box, h->st, &h->dot_work, &h->dot_out);
+    h->g64.setup(h->box, h->st, &h->dot_work, &h->dot_out, &h->cells);
   // pressure normalization weights: int psi_i (unit mass applied to ones)
   {
     LevelDesc Lu = h->Ltop();
@@ -1596,6 +1614,7 @@ void set_viscosity(mfs_handle *h, const double *eta_qp, int averaging) {
   h->active_per_qp = (averaging == MFS_AVERAGE_NONE || q1) ? 1 : 0;
   const long long na = L.ntiles_total * h->ct * (h->active_per_qp ? h->nq : 1);
   if (h->eta_active.n != na) h->eta_active.alloc(na);
+  if (!h->active_per_qp) h->cells.attach<double>(h->L[h->top], h->top, h->L[0], h->top + 1, h->st);
   v_fill<double>(h->eta_active.p, 1.0, na, h->st);
   if (q1) {
     // Q1 coefficients on every level, active table = clamped values at the

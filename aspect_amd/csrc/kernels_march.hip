@@ -159,11 +159,11 @@ struct CellIntegrals {
   const LevelDesc &L;
   // int d_a phi_m d_b phi_q over the cell
   long double grad(int a, int b, int m, int q) const {
+    const int mi[3] = {m % 3, m / 3 % 3, m / 9}, qi[3] = {q % 3, q / 3 % 3, q / 9};
+    if (mi[a] == 1 || qi[b] == 1) return 0;
     long double v = (long double)L.vol * L.ih[a] * L.ih[b];
-    for (int e = 0, s = 1; e < L.dim; ++e, s *= 3) {
-      const int i = m / s % 3, j = q / s % 3;
-      v *= e == a ? (e == b ? kK[i][j] : kD[i][j]) : (e == b ? kD[j][i] : kM[i][j]);
-    }
+    for (int e = 0; e < L.dim; ++e)
+      v *= e == a ? (e == b ? kK[mi[e]][qi[e]] : kD[mi[e]][qi[e]]) : (e == b ? kD[qi[e]][mi[e]] : kM[mi[e]][qi[e]]);
     return v;
   }
   // entry (component c, mode m), (component d, mode q) of the A block at viscosity 1
@@ -185,38 +185,35 @@ struct CellIntegrals {
   }
 };
 
-template <typename T>
-void cell_tables2(const CellIntegrals &I, std::vector<T> &out) {
-  out.assign(2 * March2::STRIDE, (T)0);
+void cell_tables2(const CellIntegrals &I, std::vector<long double> &out) {
+  out.assign(2 * March2::STRIDE, 0);
   for (int c = 0; c < 2; ++c) {
-    T *at = out.data() + c * March2::STRIDE;
+    long double *at = out.data() + c * March2::STRIDE;
     for (int r = 0; r < 2; ++r)
       for (int q = 0; q < March2::NM; ++q)
         for (int m = 0; m < March2::NM; ++m)
-          if (couples2(c, (c + r) % 2, m, q)) *at++ = (T)I.block(c, m, (c + r) % 2, q);
-    for (int m = 0; m < March2::NM; ++m) *at++ = (T)I.bt(c, m, pressure_mode2(c, m));
+          if (couples2(c, (c + r) % 2, m, q)) *at++ = I.block(c, m, (c + r) % 2, q);
+    for (int m = 0; m < March2::NM; ++m) *at++ = I.bt(c, m, pressure_mode2(c, m));
   }
 }
-template <typename T>
-void cell_tables3(const CellIntegrals &I, std::vector<T> &out) {
-  out.assign(3 * March3::STRIDE, (T)0);
+void cell_tables3(const CellIntegrals &I, std::vector<long double> &out) {
+  out.assign(3 * March3::STRIDE, 0);
   for (int c = 0; c < 3; ++c) {
-    T *const row = out.data() + c * March3::STRIDE;
+    long double *const row = out.data() + c * March3::STRIDE;
     for (int r = 0; r < 3; ++r)
       for (int k = 0; k < 8; ++k) {
         const int in = class_at(0, r, k), to = class_out(0, r, in);
         const bool c0 = r == 0 && k == 0;
-        T *at = row + class_lane(r, k);
+        long double *at = row + class_lane(r, k);
         for (int i = 0; i < (c0 ? 7 : class_size(in)); ++i)
           for (int o = 0; o < (c0 && i > 3 ? 4 : class_size(to)); ++o)
-            *at++ = (T)I.block(c, mode_from0(c, class_mode(to, c0 ? class0_out(i, o) : o)), (c + r) % 3,
-                               mode_from0(c, class_mode(in, c0 ? class0_in(i) : i)));
+            *at++ = I.block(c, mode_from0(c, class_mode(to, c0 ? class0_out(i, o) : o)), (c + r) % 3,
+                            mode_from0(c, class_mode(in, c0 ? class0_in(i) : i)));
       }
     for (int k = 0; k < 8; ++k) {
       const int cls = class_at(0, 0, k), s = cls ^ 1;  // pressure mode, numbered from direction c on
       for (int j = 0; j < class_size(cls); ++j)
-        row[16 * March3::ROWS + bt_lane(k) + j] =
-            (T)I.bt(c, mode_from0(c, class_mode(cls, j)), (s << c | s << c >> 3) & 7);
+        row[16 * March3::ROWS + bt_lane(k) + j] = I.bt(c, mode_from0(c, class_mode(cls, j)), (s << c | s << c >> 3) & 7);
     }
   }
 }
@@ -225,17 +222,29 @@ void cell_tables3(const CellIntegrals &I, std::vector<T> &out) {
 
 bool march_level(const LevelDesc &L) { return L.k == 2; }
 template <typename T>
-std::vector<T> march_tables(const LevelDesc &L) {
-  const CellIntegrals I{L};
-  std::vector<T> t;
-  if (L.dim == 3)
-    cell_tables3<T>(I, t);
+std::vector<T> march_tables(const LevelDesc &L0, int n_levels) {
+  const CellIntegrals I{L0};
+  std::vector<long double> base;
+  if (L0.dim == 3)
+    cell_tables3(I, base);
   else
-    cell_tables2<T>(I, t);
+    cell_tables2(I, base);
+  // cells of the next level have half the extents: powers of two, so that every
+  // level's entries are those of its own integrals to the last bit
+  const size_t stride = L0.dim == 3 ? March3::STRIDE : March2::STRIDE, bt = stride - (L0.dim == 3 ? 32 : March2::NM);
+  std::vector<T> t(base.size() * n_levels);
+  T *out = t.data();
+  for (int l = 0; l < n_levels; ++l) {
+    const long double fa = std::ldexp(1.0L, l * (2 - L0.dim)), fb = std::ldexp(1.0L, l * (1 - L0.dim));
+    for (const long double *p = base.data(); p != base.data() + base.size(); p += stride) {
+      for (size_t i = 0; i < bt; ++i) *out++ = (T)(p[i] * fa);
+      for (size_t i = bt; i < stride; ++i) *out++ = (T)(p[i] * fb);
+    }
+  }
   return t;
 }
-template std::vector<double> march_tables<double>(const LevelDesc &);
-template std::vector<float> march_tables<float>(const LevelDesc &);
+template std::vector<double> march_tables<double>(const LevelDesc &, int);
+template std::vector<float> march_tables<float>(const LevelDesc &, int);
 
 namespace {
 

@@ -198,13 +198,13 @@ bool launch_ablock_cheb(const LevelDesc &L, T *x, const T *b, const T *eta, int 
 // (FP64) and A-block applies in one launch from the level's cell matrices, and
 // the A-block residual fused with a Jacobi-Chebyshev step, x_out = x_in + d
 // (x_out != x_in).  false (nothing launched) where the level, the viscosity
-// table or an in-place call does not fit; march_tables: the table behind
-// LevelDesc::kmat.
+// table or an in-place call does not fit; march_tables: the tables behind
+// LevelDesc::kmat of a box's levels, one after the other, from its level 0.
 bool march_level(const LevelDesc &L);
 template <typename T>
 bool march_fits(const LevelDesc &L, int eta_per_qp);
 template <typename T>
-std::vector<T> march_tables(const LevelDesc &L);
+std::vector<T> march_tables(const LevelDesc &L0, int n_levels);
 template <typename T>
 bool launch_march(Op op, Mode mode, const LevelDesc &L, const T *src_u, const T *src_p, const T *eta, int eta_per_qp,
                   const T *rhs_u, const T *rhs_p, T *dst_u, T *dst_p, hipStream_t st);

@@ -69,6 +69,33 @@ def test_stokes_2d_matches_oracle(n):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("coarse", [(2, 1, 3), (3, 5)])
+def test_tables_of_every_level(coarse, prec):
+    # made once for all levels, when the first viscosity of one value per cell comes,
+    # here after a table per quadrature point and kept over the next viscosity
+    dim, ext, bc = len(coarse), (1.0, 0.7, 1.9), (0, 2, 1, 0, 0, 1)
+    p = O.make_problem(dim, 2, coarse + (1,) * (3 - dim), 3, ext, bc[:2 * dim], pressure_scaling=1.3, compressible=True)
+    h = StokesMatrixFreeHandler(make_box(dim, 2, coarse, 3, ext[:dim], bc[:2 * dim], True, 1.3), prec)
+    rng = np.random.default_rng(5)
+    cells = O.sizes(p, 2)["cells"]
+    h.assemble(np.exp(rng.normal(size=(cells, h.n_qp))), "project to Q1 only viscosity")
+    h.build_preconditioner()
+    for _ in range(2):
+        eta = np.exp(rng.normal(scale=2.0, size=(cells, h.n_qp)))
+        h.assemble(eta, "harmonic")
+        h.build_preconditioner()
+        levels = O.level_viscosity(p, 1.0 / np.mean(1.0 / eta, axis=1))
+        for l in range(3):
+            x = rng.normal(size=O.sizes(p, l)["nu"])
+            x = x if prec == "fp64" else x.astype(np.float32).astype(float)
+            ref = O.ablock_vmult(p, l, levels[l], x)
+            assert np.linalg.norm(h.ablock_vmult(l, x) - ref) < TOL[prec] * np.linalg.norm(ref), l
+        x = rng.normal(size=O.sizes(p, 2)["nu"] + O.sizes(p, 2)["np"])
+        ref = O.stokes_vmult(p, 2, levels[2], x)
+        assert np.linalg.norm(h.stokes_vmult(x) - ref) < TOL["fp64"] * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("compressible", [False, True])
 @pytest.mark.parametrize("n", [(9, 8, 10), (40, 33, 24), (1, 1, 1), (17, 9), (50, 3)])
 def test_constant_velocity_has_no_strain(n, compressible, prec):
