@@ -208,18 +208,19 @@ struct GMG {
   // whenever those change
   bool graphs = true;
   hipGraphExec_t vexec[2] = {nullptr, nullptr};
-  // A-block applies in the V-cycle run as two launches over all tiles through
-  // this work array (per-cell contributions, then node-wise sums) instead of
-  // eight tile colours: on coarse levels a colour launch is bound by the latency
-  // of one tile, and on the fine level the work-array traffic costs less than
-  // the colour tails and the in-kernel gather
-  // (levels with viscosities at the quadrature points, and in-place calls;
-  // set_eta_q1 allocates it before a V-cycle is captured)
+  // A-block applies that the cell-matrix kernels do not take run as two launches
+  // over all tiles through this work array (per-cell contributions, then node-wise
+  // sums) instead of eight tile colours: on coarse levels a colour launch is bound
+  // by the latency of one tile, and on the fine level the work-array traffic costs
+  // less than the colour tails and the in-kernel gather.  These are levels with
+  // viscosities at the quadrature points (set_eta_q1 makes it large enough for all
+  // of them before a V-cycle is captured), the eigenvalue estimate of level 0, and
+  // in-place calls, each with its level's size (128^3 in double: 573 MB)
   DBuf<T> swork;
   T *split_for(int l) {
     const LevelDesc &L = lv[l]->L;
     if (laplace || split_work_size(L) == 0) return nullptr;
-    if (swork.n < split_work_size(L)) swork.alloc(split_work_size(lv[top]->L));
+    if (swork.n < split_work_size(L)) swork.alloc(split_work_size(L));
     return swork.p;
   }
   bool ietan_ok = false;  // GMGLevel::ietan matches the current level viscosity

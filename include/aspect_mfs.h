@@ -283,7 +283,8 @@ int mfs_correct_stokes_rhs(mfs_handle *h, const double *u0, double *rhs);
 
 /* Device-resident variants: all pointers are device pointers. */
 int mfs_stokes_vmult_device(mfs_handle *h, const double *d_src, double *d_dst);
-/* Level A-block apply in the GMG precision (float or double device arrays). */
+/* Level A-block apply in the GMG precision (float or double device arrays).
+ * The first call in place on a level allocates its work array. */
 int mfs_ablock_vmult_device(mfs_handle *h, int level, const void *d_src, void *d_dst);
 /* Allocation-free variant of mfs_ablock_vmult_device.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under

@@ -112,6 +112,19 @@ def test_constant_velocity_has_no_strain(n, compressible, prec):
     assert bool((y == 0).all())
 
 
+def test_set_up_of_cellwise_levels_keeps_no_work_array():
+    # the estimate of level 0 runs the split form: its work array has that
+    # level's size, not the finest one's (72 MB here)
+    for n in (8, 64):  # the first handle pays what the process pays once
+        h = StokesMatrixFreeHandler(make_box(3, 2, (1, 1, 1), n.bit_length(), (1.0,) * 3, (1,) * 6), "fp64")
+        h.assemble(np.ones((n ** 3, h.n_qp)), "harmonic")
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        h.build_preconditioner()
+        used = before - torch.cuda.mem_get_info()[0]
+    assert used < 16 << 20  # the inverse cell viscosities: 2.4 MB over the levels
+
+
 def test_source_outside_the_mesh_is_not_read_into_rows():
     # columns beyond the mesh read the nearest cells and discard the values:
     # an infinity at one node reaches only the rows of the cells that hold it
