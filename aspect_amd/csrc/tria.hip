@@ -834,6 +834,7 @@ namespace {
 // lanes to a row 7.3, 5.7 and 5.8 us).  A row's entries are a multiple of the 8 (Q1)
 // or 27 (Q2) nodes of a cell, so more lanes would idle on the prolongation's.
 constexpr int SPMV_LANES = 16;
+constexpr long long SPMV_ROWS = 1LL << 27;
 __global__ void k_spmv(const long long rows, const long long *__restrict__ ptr, const long long *__restrict__ col,
                        const double *__restrict__ val, const double *__restrict__ x, double *__restrict__ y,
                        const int add) {
@@ -934,7 +935,12 @@ struct DevCsr {
   }
   void apply(const double *x, double *y, bool add, hipStream_t st) const {
     if (rows <= 0) return;
-    hipLaunchKernelGGL(k_spmv, dim3(nblk(rows * SPMV_LANES)), dim3(256), 0, st, rows, ptr.p, col.p, val.p, x, y, add ? 1 : 0);
+    // a launch holds less than 2^32 threads: rows in parts
+    for (long long r = 0; r < rows; r += SPMV_ROWS) {
+      const long long n = std::min(rows - r, SPMV_ROWS);
+      hipLaunchKernelGGL(k_spmv, dim3(nblk(n * SPMV_LANES)), dim3(256), 0, st, n, ptr.p + r, col.p, val.p, x, y + r,
+                         add ? 1 : 0);
+    }
     MFS_HIP(hipGetLastError());
   }
 };
