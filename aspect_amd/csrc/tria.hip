@@ -105,15 +105,31 @@ __device__ __forceinline__ int component_of(long long dof, long long nn) {
   return (dof >= nn ? 1 : 0) + (dof >= 2 * nn ? 1 : 0);
 }
 // sums of the constrained DoFs that have masters, one thread each, for
-// k_assemble to add to the masters
-__global__ void k_line_sums(const int n, const long long nn, const long long cs, const double *__restrict__ cb,
-                            const long long *__restrict__ iptr, const int *__restrict__ ioff,
-                            const long long *__restrict__ dof, double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const long long i = dof[t];
-  const int comp = component_of(i, nn);
-  out[t] = node_sum(cb, iptr, ioff, i - comp * nn, comp * cs);
+// k_assemble to add to the masters.  The Stokes operator's two blocks share a
+// launch: with one each, meshes with short lists (2D shell, 4.9k cells: 22.8 us
+// an apply with the lists summed by the masters, 23.8 us) were slower
+struct LineSums {
+  int n;
+  long long nn, cs;
+  const double *cb;
+  const long long *iptr;
+  const int *ioff;
+  const long long *dof;
+  double *out;
+};
+__device__ __forceinline__ void line_sum(const LineSums &b, int t) {
+  if (t >= b.n) return;
+  const long long i = b.dof[t];
+  const int comp = component_of(i, b.nn);
+  b.out[t] = node_sum(b.cb, b.iptr, b.ioff, i - comp * b.nn, comp * b.cs);
+}
+__global__ void k_line_sums(const LineSums b) { line_sum(b, blockIdx.x * blockDim.x + threadIdx.x); }
+// the first nb blocks of threads sum for u, the others for p
+__global__ void k_line_sums2(const unsigned nb, const LineSums u, const LineSums p) {
+  if (blockIdx.x < nb)
+    line_sum(u, blockIdx.x * blockDim.x + threadIdx.x);
+  else
+    line_sum(p, (blockIdx.x - nb) * blockDim.x + threadIdx.x);
 }
 
 // dst[i] for the DoFs of one block (nn nodes per component, component stride
@@ -540,6 +556,19 @@ struct mfs_tria {
     hipLaunchKernelGGL(k_resolve, dim3(nb), dim3(256), 0, s, c.n, src, c.row.p, c.off.p, c.mas.p, c.w.p, out);
     MFS_HIP(hipGetLastError());
   }
+  // before the assemble of the blocks written
+  void line_sums(bool wr_u, bool wr_p, hipStream_t s) {
+    LineSums u{}, p{};
+    if (wr_u) u = {con_u.n_hang, nn_u, (long long)nv * CT, cbu.p, iptr_u.p, ioff_u.p, con_u.hang.p, con_u.sums.p};
+    if (wr_p) p = {con_p.n_hang, nn_p, 0, cbp.p, iptr_p.p, ioff_p.p, con_p.hang.p, con_p.sums.p};
+    const unsigned nu = (unsigned)((u.n + 63) / 64), np = (unsigned)((p.n + 63) / 64);
+    if (nu + np == 0) return;
+    if (nu == 0 || np == 0)
+      hipLaunchKernelGGL(k_line_sums, dim3(nu + np), dim3(64), 0, s, np == 0 ? u : p);
+    else
+      hipLaunchKernelGGL(k_line_sums2, dim3(nu + np), dim3(64), 0, s, nu, u, p);
+    MFS_HIP(hipGetLastError());
+  }
   void assemble(const double *cb, long long nn, long long cs, const Buf<long long> &ip, const Buf<int> &io,
                 DevCon &c, const double *src, double *dst, int ident, hipStream_t s, int mode = AS_SET,
                 const ChebStep &ch = ChebStep{}) {
@@ -547,9 +576,6 @@ struct mfs_tria {
     // below 256 blocks of 256, and chains of gathers end sooner spread over more CUs (12-iteration solve on
     // 1843 cells 25.0 -> 23.7 ms, Stokes apply on 14.7k cells 80 -> 78 us)
     const unsigned nb = (unsigned)((c.n + 63) / 64);
-    if (c.n_hang > 0)
-      hipLaunchKernelGGL(k_line_sums, dim3((unsigned)((c.n_hang + 63) / 64)), dim3(64), 0, s, c.n_hang, nn, cs, cb, ip.p,
-                         io.p, c.hang.p, c.sums.p);
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(nb), dim3(64), 0, s, c.n, nn, cs, cb, ip.p, io.p, c.row.p, c.tptr.p, c.tline.p,
                          c.tw.p, c.sums.p, src, dst, ident, ch);
@@ -570,6 +596,7 @@ struct mfs_tria {
     if (kind == 0) {
       resolve(x, xu.p, con_u, s);
       launch_cells<double>(OP_ABLOCK, L, nbatch, xu.p, nullptr, eta.p, cbu.p, cbp.p, s);
+      line_sums(true, false, s);
       assemble(cbu.p, nn_u, (long long)nv * CT, iptr_u, ioff_u, con_u, x, dst, 1, s, mode, ch);
       return;
     }
@@ -582,6 +609,7 @@ struct mfs_tria {
       hipLaunchKernelGGL(k_tria_mass_apply<2>, dim3(nb), dim3(64), 0, s, ncells, cell_p.p, mass_mat.p, x,
                          con_p.row.p, con_p.off.p, con_p.mas.p, con_p.w.p, cbp.p);
     MFS_HIP(hipGetLastError());
+    line_sums(false, true, s);
     assemble(cbp.p, nn_p, 0, iptr_p, ioff_p, con_p, x, dst, 1, s, mode, ch);
   }
 
@@ -621,6 +649,7 @@ struct mfs_tria {
     } else {
       launch_cells<double>((Op)op, L, nbatch, rd_u ? xu.p : nullptr, rd_p ? xp.p : nullptr, eta.p, cbu.p, cbp.p, s);
     }
+    line_sums(wr_u, wr_p, s);
     if (wr_u)
       assemble(cbu.p, nn_u, (long long)nv * CT, iptr_u, ioff_u, con_u, su, du, (op == MFS_OP_BT || plain) ? 0 : 1, s);
     if (wr_p) assemble(cbp.p, nn_p, 0, iptr_p, ioff_p, con_p, sp, dp, plain ? 0 : 1, s);

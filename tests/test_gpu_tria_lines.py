@@ -41,3 +41,18 @@ def test_many_lines_on_one_master(mesh, n_slaves):
     for got, want in ((gpu.vmult("ablock", u), ref.ablock(u)), (gpu.vmult("mass", p), ref.mass(p)),
                       (gpu.vmult("bt", p), ref.bt(p))):
         assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("n_u,n_p", [(0, 0), (1, 0), (0, 1), (63, 2), (64, 9), (65, 1)])
+def test_stokes_with_lines_in_either_block(n_u, n_p):
+    # both blocks' line sums in one launch, split at a whole block of 64 threads
+    m = T.Tria(T.BoxCoarse(3, (4, 3, 2), (1.5, 1.0, 1.2)), 1).build({})
+    rng = np.random.default_rng(n_u)
+    m.con_u, m.con_p = lines(m.n_dofs_u, n_u, rng), lines(m.n_dofs_p, n_p, rng)
+    print("stokes lines", n_u, n_p, flush=True)
+    eta = np.exp(rng.normal(size=(m.n_cells, 27)))
+    ref, gpu = OT.Operators(m, eta), TriaOperators(m)
+    gpu.set_viscosity(eta)
+    x = rng.normal(size=m.n_dofs_u + m.n_dofs_p)
+    got, want = gpu.vmult("stokes", x), ref.stokes(x)
+    assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
