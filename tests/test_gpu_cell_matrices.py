@@ -12,9 +12,12 @@ from aspect_amd import StokesMatrixFreeHandler, make_box
 pytestmark = pytest.mark.gpu
 
 MIXED = (1, 2, 0, 1, 1, 2)
-# a box owns 7 x 7 columns of cells or a longer strip, a march 1 to 11 layers:
-# one cell, one short of / exactly / one past a box, strips, several marches
+# a box owns 7 x 7 columns of cells or a longer strip, small levels march one layer:
+# one cell, one short of / exactly / one past a box, strips
 SIZES = [(1, 1, 1), (6, 7, 8), (7, 8, 2), (8, 6, 13), (21, 2, 3), (2, 30, 5), (15, 14, 12), (40, 33, 24)]
+# larger levels march up to 11 layers in double and 6 in single, with and without a rest
+LONG = [(56, 100, 3), (56, 100, 6), (64, 72, 12), (56, 100, 14), (56, 64, 33), (100, 120, 10), (72, 72, 33), (56, 64, 45),
+        (64, 64, 41)]
 # a row sums at most 8 cells x 36 products after 6 sums: ~ sqrt(8 * 42) rounding errors of the largest
 # terms, which the smooth part of a random field leaves ~ 10 times larger than the row
 TOL = {"fp64": 200 * 2.0 ** -53 * 10, "fp32": 200 * 2.0 ** -24 * 10}
@@ -37,9 +40,58 @@ def _against_in_place(apply, x):
     return float((y - z).norm() / z.norm())
 
 
+def march_layers(n, size):
+    """Layers per march of the launch rule (values of size bytes)."""
+    boxes = min(-(-(n[0] + 1) // (tx - 1)) * -(-(n[1] + 1) // (64 // tx - 1)) for tx in range(3, 22))
+    best, cost = 1, None
+    for layers in (1, 2, 3, 4, 6, 8, 11)[:7 if size == 8 else 5]:
+        r = boxes * ((n[2] + layers) // layers) / (512 if size == 8 else 1024)
+        c = (np.ceil(r) if r < 3 else r + 0.5) * (layers + 1.5)
+        if cost is None or c < cost:
+            best, cost = layers, c
+    return best
+
+
+def test_long_marches_are_reached():
+    for size, layers in ((8, {2, 3, 4, 6, 8, 11}), (4, {1, 2, 3, 4, 6})):
+        got = [(march_layers(n, size), (n[2] + 1) % march_layers(n, size) == 0) for n in LONG]
+        assert {g[0] for g in got} == layers and {g[1] for g in got if g[0] > 1} == {True, False}
+    assert all(march_layers(n, 4) == 1 for n in SIZES)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", LONG)
+def test_long_march_chebyshev_matches_quadrature(n, prec):
+    # the step fused into the march, eight times, against the recurrence with in-place applies in double
+    h, s, rng = _box(n, MIXED, True, prec)
+    q = h if prec == "fp64" else _box(n, MIXED, True, "fp64")[0]
+    print("chebyshev", n, prec, flush=True)
+    h.build_preconditioner()
+    theta, delta = h.smoother_info()[0, 0, 2:4]
+    b = rng.normal(size=s["nu"])
+    b = b if prec == "fp64" else b.astype(np.float32).astype(float)
+    bd, dinv = torch.tensor(b, device="cuda:0"), 1.0 / torch.tensor(q.ablock_diagonal(0), device="cuda:0")
+
+    def apply(x):
+        y = x.clone()
+        torch.cuda.synchronize()
+        q.ablock_vmult_device(0, y.data_ptr(), y.data_ptr())
+        q.synchronize()
+        return y
+
+    x = d = dinv * bd / theta
+    rho = delta / theta
+    for _ in range(1, 8):
+        new = 1.0 / (2.0 * theta / delta - rho)
+        d = new * rho * d + 2.0 * new / delta * dinv * (bd - apply(x))
+        x, rho = x + d, new
+    got = torch.tensor(h.chebyshev(0, 0, b), device="cuda:0")
+    assert float((got - x).norm() / x.norm()) < 8 * TOL[prec]  # an apply's error each step
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("compressible", [False, True])
-@pytest.mark.parametrize("n", SIZES + [(1, 1), (7, 7), (8, 6), (50, 3), (33, 40)])
+@pytest.mark.parametrize("n", LONG + SIZES + [(1, 1), (7, 7), (8, 6), (50, 3), (33, 40)])
 def test_ablock_apply_matches_quadrature(n, compressible, prec):
     h, s, rng = _box(n, MIXED, compressible, prec)
     print("ablock", n, prec, compressible, flush=True)
@@ -47,7 +99,7 @@ def test_ablock_apply_matches_quadrature(n, compressible, prec):
     assert _against_in_place(lambda a, b: h.ablock_vmult_device(0, a, b), x) < TOL[prec]
 
 
-@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("n", SIZES + LONG)
 def test_stokes_apply_matches_quadrature(n):
     for bc in (MIXED, (2,) * 6, (0,) * 6):
         h, s, rng = _box(n, bc, False, "fp64")
