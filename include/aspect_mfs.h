@@ -292,7 +292,9 @@ int mfs_ablock_vmult_device(mfs_handle *h, int level, const void *d_src, void *d
  * The degree-2 split apply's work array (in-tile sums of the tile-boundary
  * nodes) lives in a fixed device array of the library,
  * MFS_NOALLOC_SCRATCH_BYTES per GPU (held until the process ends), instead of
- * the handle's buffer; the call allocates and frees nothing.  Levels whose
+ * the handle's buffer; the call allocates and frees nothing.  A call with one
+ * viscosity per cell and another destination than its source reads no work
+ * array, but the limit is the level's all the same.  Levels whose
  * work array (3 x 386 values per 4^3-cell tile in 3D, 2 x 289 per 8^2-cell
  * tile in 2D) exceeds it return MFS_ERROR: at most 8149 tiles in FP64 and
  * 16299 in FP32 (80^3 and 100^3 cells) in 3D.  Degree-3 levels use no work
