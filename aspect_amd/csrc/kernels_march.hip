@@ -25,14 +25,15 @@
 // A workgroup owns the nodes of a box of cells and computes every cell that
 // touches them, so each node is finished by one thread: no work array, no
 // second pass, no atomics, one launch, fixed summation order.  The price is
-// one extra layer of cells at the low side of the box (64 columns compute 49
-// to 56 owned ones).
+// one extra layer of cells at the low side of the box (of at most 64 columns 40 to 49
+// are owned) and one below each march.
 //
 // Against the split quadrature kernels (kernels_planes.hip, kernels_gather.hip):
 // FP64 Stokes apply 96^3 417 -> 173 us, 8^3 16.7 -> 4.6 us; FP32 A block 96^3
-// 209 -> 91 us; 64^3 preconditioner 2.46 -> 2.15 ms; 2D ensemble 81 -> 49 ms.
-// Bound (96^3, FP64): 6 waves per CU hide neither the LDS exchange nor the
-// loads fully; vector ALUs are a third busy, memory moves 2.1 TB/s.
+// 209 -> 92 us; 64^3 preconditioner 2.46 -> 2.15 ms; 2D ensemble 81 -> 49 ms.
+// Bound (96^3, counters): in FP64 latency, 1.6 waves a SIMD wait 41 % of the time at
+// the two barriers of a layer and for loads; the vector units are 40 % busy and memory
+// moves 2.65 TB/s, 54 % of what a copy reaches.  In FP32 the vector units, 70 % busy.
 
 #include <hip/hip_runtime.h>
 
@@ -1001,8 +1002,7 @@ __global__ void __launch_bounds__(64)
     if (own) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (2 * cx + (q & 1) <= l0 && 2 * cy + (q >> 1) <= l1)
-{
+        if (2 * cx + (q & 1) <= l0 && 2 * cy + (q >> 1) <= l1) {
           const T val = con[d] >> (3 * (q >> 1) + (q & 1)) & 1 ? raw[d][q] : o[q >> 1][q & 1];
           finish_node<MODE, T>(val, io, vo[q >> 1][q & 1], 0, ch);
         }
@@ -1078,10 +1078,11 @@ bool overlap(const T *a, const T *b, long long n) {
   return a < b + n && b < a + n;
 }
 
+}  // namespace
+
 // what the kernels assume: degree 2 on a uniform box with its cell matrices in
 // this precision, one viscosity per cell, constrained values read as zero,
 // byte offsets in a plane and viscosity indices in 32 bits
-}  // namespace
 template <typename T>
 bool march_fits(const LevelDesc &L, int eta_per_qp) {
   return L.k == 2 && !L.geo && !L.plain_read && !eta_per_qp && L.kmat && L.kmat_size == (int)sizeof(T) &&
